@@ -127,9 +127,30 @@ bool tiled_backward_supports(const srw_desc_t& d);
 size_t tiled_backward_workspace_bytes(const srw_desc_t& d);
 hipError_t tiled_backward(const BackwardArgs& a);
 
+// Unit diagnostics (srw_mfma.hip): unit_diag[u] = (sum of the unit's scores,
+// its max gate) from part[row_blocks][N] = (sum of scores, max of s - tau, or
+// with gate_direct the max gate itself).
+hipError_t launch_unit_diag(const float2* part, int64_t row_blocks, int64_t N, float* unit_diag, const GateParams& gp,
+                            float exp_scale, bool gate_direct, hipStream_t s);
+
+// Training diagnostics of a stored score matrix (srw_diag.hip).
+struct TiledDiagArgs {
+  const uint16_t* S;   // [Tv, N64] bf16 scores (zero past N)
+  const float* tau;    // [Tv]
+  float* part;         // scratch: [ceil(N / 256)][Tv][kTokPartDiag]
+  float2* unit_part;   // [ceil(Tv / 32)][N] (sum of scores, max of s - tau) for launch_unit_diag, or null
+  float* tok_sum;      // [Tv][kTokPartDiag]: the slots from TP_SMAX on are written
+  float* token_diag;   // [Tv][SRW_TDIAG_COUNT]: SUM_S3 and SUM_S4 are written; or null
+  int64_t Tv, N, N64;
+  GateParams gp;
+  float exp_scale;     // -sharpness * log2(e)
+};
+hipError_t tiled_diag(const TiledDiagArgs& a, hipStream_t s);
+
 // Tiled-GEMM kernels for wide layers (bf16), see srw_tiled.hip: P = gated
 // product materialised in HBM; d_model and d_route multiples of 64.
 bool tiled_supports(const srw_desc_t& d);
+bool tiled_diag_supports(const srw_desc_t& d);  // with SRW_FLAG_DIAG
 size_t tiled_workspace_bytes(const srw_desc_t& d);
 bool tiled_runs_sparse(const srw_desc_t& d);  // SRW_FLAG_SPARSE_SKIP at a width the sparse kernels take
 hipError_t tiled_forward(const LaunchArgs& a);

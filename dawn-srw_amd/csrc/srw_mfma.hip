@@ -48,49 +48,6 @@ constexpr int kTokTile = 128;     // tokens per workgroup
 constexpr int kUnitTile = 32;     // units per tile
 constexpr int kTargetBlocks = 256;
 
-// Lane exchanges within 32-lane halves, on the vector ALU (DPP and the gfx950
-// row swap) rather than the LDS crossbar: the value of lane (lane ^ m).
-__device__ inline float as_f(int v) { return __builtin_bit_cast(float, v); }
-__device__ inline int as_i(float v) { return __builtin_bit_cast(int, v); }
-template <int M>
-__device__ inline float lane_xor(float v, int lane) {
-  if constexpr (M == 1) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0xB1, 0xF, 0xF, true));  // quad_perm [1,0,3,2]
-  if constexpr (M == 2) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x4E, 0xF, 0xF, true));  // quad_perm [2,3,0,1]
-  if constexpr (M == 4) {
-    const float up = as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x104, 0xF, 0xF, true));  // row_shl:4
-    const float dn = as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x114, 0xF, 0xF, true));  // row_shr:4
-    return (lane & 4) ? dn : up;
-  }
-  if constexpr (M == 8) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x128, 0xF, 0xF, true));  // row_ror:8
-  if constexpr (M == 16) {
-    const auto r = __builtin_amdgcn_permlane16_swap(as_i(v), as_i(v), false, false);
-    return as_f((lane & 16) ? r[0] : r[1]);
-  }
-}
-
-// Reduce-scatter of 16 values per lane over the 32 lanes of each half: on
-// return a[0] of lane l holds the reduction, over the half's 32 lanes, of
-// element k = 8 (l & 1) + 4 (l >> 1 & 1) + 2 (l >> 2 & 1) + (l >> 3 & 1).
-template <class Op>
-__device__ inline void reduce_scatter16(float (&a)[16], int lane, Op op) {
-  auto step = [&](auto mtag, int cnt) {
-    constexpr int M = decltype(mtag)::value;
-    const bool up = lane & M;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if (k >= cnt / 2) break;
-      const float send = up ? a[k] : a[k + cnt / 2], keep = up ? a[k + cnt / 2] : a[k];
-      a[k] = op(keep, lane_xor<M>(send, lane));
-    }
-  };
-  step(std::integral_constant<int, 1>{}, 16);
-  step(std::integral_constant<int, 2>{}, 8);
-  step(std::integral_constant<int, 4>{}, 4);
-  step(std::integral_constant<int, 8>{}, 2);
-  a[0] = op(a[0], lane_xor<16>(a[0], lane));
-}
-
-
 // A 32-row tile of a row-major bf16 [rows, K] array (E or R), staged in LDS
 // as K / 16 one-KB blocks.  Load block j moves whole 128-byte lines (8 rows x
 // 128 B; 16 rows x 64 B when K = 32): a wave load that touches 32 B of each of
@@ -583,11 +540,6 @@ __global__ __launch_bounds__(kThreads) void srw_stats_batch_kernel(Batch<StatsPa
 // ---------------------------------------------------------------------------
 // main: fused score / read / gate / write for one (token tile, N-split).
 // ---------------------------------------------------------------------------
-// Per-token partial slots of the main kernel with diagnostics (kTokPartDiag
-// floats per (split, row)); slots 0-2 are sum gate, sum intensity, active count.
-constexpr int kTokPartDiag = 12;
-enum { TP_SMAX = 4, TP_STRONG, TP_BOUND, TP_075, TP_030, TP_CAP, TP_GLOGG };
-
 // Rows of the main kernel are "virtual tokens" v = t * routes + r: h, tau,
 // outputs and every partial are indexed by v, x by v / routes (paired QK runs
 // as 2T rows sharing each x row).
@@ -3400,14 +3352,15 @@ hipError_t mfma_forward(const LaunchArgs& a, const char** path_name) {
   }
   // finalize
   if ((e = launch_finalize(f, a.stream)) != hipSuccess) return e;
-  if (unit_part) {
-    const int64_t rows = (g.T + 31) / 32;
-    hipLaunchKernelGGL(srw_unit_diag_kernel, dim3(static_cast<unsigned>((d.n_units + 63) / 64)), dim3(256), 0,
-                       a.stream, unit_part, rows, static_cast<int64_t>(d.n_units), unit_diag, a.gp, f.exp_scale,
-                       gl ? 1 : 0);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  if (unit_part) return launch_unit_diag(unit_part, (g.T + 31) / 32, d.n_units, unit_diag, a.gp, f.exp_scale, gl, a.stream);
   return hipSuccess;
+}
+
+hipError_t launch_unit_diag(const float2* part, int64_t row_blocks, int64_t N, float* unit_diag, const GateParams& gp,
+                            float exp_scale, bool gate_direct, hipStream_t s) {
+  hipLaunchKernelGGL(srw_unit_diag_kernel, dim3(static_cast<unsigned>((N + 63) / 64)), dim3(256), 0, s, part,
+                     row_blocks, N, unit_diag, gp, exp_scale, gate_direct ? 1 : 0);
+  return hipGetLastError();
 }
 
 hipError_t launch_tau(const float* mom, const float* tau_off, float* tau, int64_t T, int S_st, int64_t N, int ms,

@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace srw {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -69,6 +71,71 @@ __device__ inline void barrier_lds() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Lane exchanges within 32-lane halves, on the vector ALU (DPP and the gfx950
+// row swap) rather than the LDS crossbar: the value of lane (lane ^ m).
+__device__ inline float as_f(int v) { return __builtin_bit_cast(float, v); }
+__device__ inline int as_i(float v) { return __builtin_bit_cast(int, v); }
+template <int M>
+__device__ inline float lane_xor(float v, int lane) {
+  if constexpr (M == 1) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0xB1, 0xF, 0xF, true));  // quad_perm [1,0,3,2]
+  if constexpr (M == 2) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x4E, 0xF, 0xF, true));  // quad_perm [2,3,0,1]
+  if constexpr (M == 4) {
+    const float up = as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x104, 0xF, 0xF, true));  // row_shl:4
+    const float dn = as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x114, 0xF, 0xF, true));  // row_shr:4
+    return (lane & 4) ? dn : up;
+  }
+  if constexpr (M == 8) return as_f(__builtin_amdgcn_mov_dpp(as_i(v), 0x128, 0xF, 0xF, true));  // row_ror:8
+  if constexpr (M == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(as_i(v), as_i(v), false, false);
+    return as_f((lane & 16) ? r[0] : r[1]);
+  }
+}
+
+// Reduce-scatter of 16 values per lane over the 32 lanes of each half: on
+// return a[0] of lane l holds the reduction, over the half's 32 lanes, of
+// element k = 8 (l & 1) + 4 (l >> 1 & 1) + 2 (l >> 2 & 1) + (l >> 3 & 1).
+template <class Op>
+__device__ inline void reduce_scatter16(float (&a)[16], int lane, Op op) {
+  auto step = [&](auto mtag, int cnt) {
+    constexpr int M = decltype(mtag)::value;
+    const bool up = lane & M;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k >= cnt / 2) break;
+      const float send = up ? a[k] : a[k + cnt / 2], keep = up ? a[k + cnt / 2] : a[k];
+      a[k] = op(keep, lane_xor<M>(send, lane));
+    }
+  };
+  step(std::integral_constant<int, 1>{}, 16);
+  step(std::integral_constant<int, 2>{}, 8);
+  step(std::integral_constant<int, 4>{}, 4);
+  step(std::integral_constant<int, 8>{}, 2);
+  a[0] = op(a[0], lane_xor<16>(a[0], lane));
+}
+
+// Per-token partial slots of the main kernel with diagnostics (kTokPartDiag
+// floats per (split, row)); slots 0-2 are sum gate, sum intensity, active count.
+constexpr int kTokPartDiag = 12;
+enum { TP_SMAX = 4, TP_STRONG, TP_BOUND, TP_075, TP_030, TP_CAP, TP_GLOGG };
+
+// The v4.1 gate of one bf16 score in the folded form (v41:503-511):
+// arg = s c + k (c = -sharpness log2 e, k = -(tau + thr) c), act = 1 / (1 +
+// 2^arg), intensity = eps + min(max(s - tau - thr - cut, 0), maxi), g = act
+// intensity; the sign bit of arg is the pass bit.  The product stays a
+// rounded multiply (no contraction into a caller's running sum), so the
+// dense gate kernel and the sparse mark kernel sum the same gate values.
+struct GateElem {
+  float g, inten;
+  uint32_t sign;
+};
+__device__ inline GateElem gate_elem(float s, float c_exp, float k_exp, float tau_cut, float eps, float maxi) {
+#pragma clang fp contract(off)
+  const float arg = fmaf(s, c_exp, k_exp);
+  const float act = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
+  const float inten = eps + __builtin_amdgcn_fmed3f(s - tau_cut, 0.0f, maxi);
+  return GateElem{act * inten, inten, __float_as_uint(arg)};
 }
 
 // v4.0.1 GELU gate of a score s (v401:303-306): z = (s - tau) / s_std,

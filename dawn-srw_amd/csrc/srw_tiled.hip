@@ -322,24 +322,6 @@ struct TGateParams {
   float exp_scale;       // -sharpness * log2(e)
 };
 
-// The v4.1 gate of one bf16 score in the folded form (v41:503-511):
-// arg = s c + k (c = -sharpness log2 e, k = -(tau + thr) c), act = 1 / (1 +
-// 2^arg), intensity = eps + min(max(s - tau - thr - cut, 0), maxi), g = act
-// intensity; the sign bit of arg is the pass bit.  The product stays a
-// rounded multiply (no contraction into a caller's running sum), so the
-// dense gate kernel and the sparse mark kernel sum the same gate values.
-struct GateElem {
-  float g, inten;
-  uint32_t sign;
-};
-__device__ inline GateElem gate_elem(float s, float c_exp, float k_exp, float tau_cut, float eps, float maxi) {
-#pragma clang fp contract(off)
-  const float arg = fmaf(s, c_exp, k_exp);
-  const float act = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
-  const float inten = eps + __builtin_amdgcn_fmed3f(s - tau_cut, 0.0f, maxi);
-  return GateElem{act * inten, inten, __float_as_uint(arg)};
-}
-
 // KEEP (the backward's recompute): P and x.r go to P_out / XR_out and the
 // stored scores stay.  GOUT: every unit's fp32 gate also goes to G (a
 // variant of its own: the per-element stores and their addresses would
@@ -980,8 +962,10 @@ __global__ __launch_bounds__(kGThreads) void tiled_write_batch_kernel(TWriteBatc
 // sum[t] = sum over s of part[s][t] (sum gate, sum intensity, active count).
 // 64 tokens per workgroup, four partial groups s = g mod 4 per token with
 // eight loads in flight each, combined in LDS.
+// ss: floats per row of sum (4, or kTokPartDiag with diagnostics, whose
+// kernel fills the other slots).
 __global__ __launch_bounds__(256) void tiled_tok_sum_kernel(const float* __restrict__ part, float* __restrict__ sum,
-                                                            int64_t Tv, int S) {
+                                                            int64_t Tv, int S, int ss) {
   __shared__ float4 red[4][64];
   const int c = threadIdx.x & 63, grp = threadIdx.x >> 6;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + c;
@@ -1022,7 +1006,7 @@ __global__ __launch_bounds__(256) void tiled_tok_sum_kernel(const float* __restr
       r.z += red[g][c].z;
     }
     r.w = 0.f;
-    *reinterpret_cast<float4*>(sum + t * 4) = r;
+    *reinterpret_cast<float4*>(sum + t * ss) = r;
   }
 }
 
@@ -1064,7 +1048,7 @@ TGeo tgeo(const srw_desc_t& d) {
 }
 
 struct TLayout {
-  size_t wt, P, mom, tau, out_part, tok_part, tok_sum, uni, list, glist, cstart, G, total;
+  size_t wt, P, mom, tau, out_part, tok_part, tok_sum, uni, list, glist, cstart, G, diag, upart, total;
 };
 
 // sparse skip at prefill sizes: the gathered GEMMs' widths (D = 256 F; a
@@ -1072,7 +1056,8 @@ struct TLayout {
 // R and W rows addressed by 32-bit byte offsets
 bool sparse_width_ok(int64_t D) { return D == 256 || D == 512 || D == 1024; }
 bool tiled_sparse(const srw_desc_t& d) {
-  return (d.flags & SRW_FLAG_SPARSE_SKIP) && !(d.flags & SRW_FLAG_GATE_OUT) && sparse_width_ok(d.d_model) &&
+  return (d.flags & SRW_FLAG_SPARSE_SKIP) && !(d.flags & (SRW_FLAG_GATE_OUT | SRW_FLAG_DIAG)) &&
+         sparse_width_ok(d.d_model) &&
          d.n_units * d.d_model * 2 < (int64_t(1) << 32);
 }
 
@@ -1091,8 +1076,14 @@ TLayout tlayout(const srw_desc_t& d, const TGeo& g) {
   off += al256(static_cast<int64_t>(g.S) * g.Tv * d.d_model * 4);
   l.tok_part = off;
   off += al256(static_cast<int64_t>(2 * g.CT) * g.Tv * 4 * 4);
+  const bool dg = (d.flags & SRW_FLAG_DIAG) != 0;
   l.tok_sum = off;
-  off += al256(g.Tv * 4 * 4);
+  off += al256(g.Tv * (dg ? kTokPartDiag : 4) * 4);
+  // diagnostics: per 256-unit slice and row, per 32-row block and unit (TiledDiagArgs)
+  l.diag = off;
+  if (dg) off += al256(static_cast<int64_t>(g.CT) * g.Tv * kTokPartDiag * 4);
+  l.upart = off;
+  if (dg) off += al256((g.Tv + 31) / 32 * g.N * static_cast<int64_t>(sizeof(float2)));
   // sparse skip: per 32-token tile the union words, the unit list and the
   // units' slots in G, the chunk starts, and G (256 CT slots of 32 gates)
   l.uni = l.list = l.glist = l.cstart = l.G = off;
@@ -1118,6 +1109,18 @@ hipError_t set_lds(const void* fn, int bytes = kGemmLds) {
 // 32 bits: 256 rows of ld bf16 elements must stay below 4 GiB (ld = N or T
 // padded to 64 for the stored [., N64] / [., T64] arrays).
 static bool tile_offsets_fit(int64_t ld) { return 256 * ((ld + kNAlign - 1) / kNAlign * kNAlign) * 2 < (int64_t(1) << 32); }
+
+// Diagnostics come from the stored scores before the gate kernel writes P
+// over them.  They take the maxima of gate and intensity at the max score, so
+// the constants must keep both non-decreasing in the score, and pass bits
+// from the sign of the margin (sharpness > 0).
+bool tiled_diag_supports(const srw_desc_t& d) {
+  if (!(d.flags & SRW_FLAG_DIAG) || d.stats_mode != SRW_STATS_ONEPASS) return false;
+  if (!(d.sharpness > 0.f) || !(d.epsilon >= 0.f) || !(d.max_intensity >= 0.f)) return false;
+  srw_desc_t plain = d;
+  plain.flags &= ~SRW_FLAG_DIAG;
+  return tiled_supports(plain);
+}
 
 bool tiled_supports(const srw_desc_t& d) {
   if (d.dtype != SRW_BF16 || d.gate != SRW_GATE_V41) return false;
@@ -1173,7 +1176,7 @@ hipError_t tiled_sparse_rest(const LaunchArgs& a, const TGeo& g, const TLayout& 
   hipLaunchKernelGGL(sp_mark_kernel, dim3(static_cast<unsigned>(TT32 * sgroups)), dim3(256), 0, a.stream, mp);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(tiled_tok_sum_kernel, dim3(static_cast<unsigned>((g.Tv + 63) / 64)), dim3(256), 0, a.stream,
-                     tok_part, tok_sum, g.Tv, 2 * g.CT);
+                     tok_part, tok_sum, g.Tv, 2 * g.CT, 4);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(sp_list_kernel, dim3(static_cast<unsigned>(TT32)), dim3(256), 0, a.stream, uni, W32, g.N, g.cs,
                      g.nc, list, glist, cstart);
@@ -1264,10 +1267,33 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   if ((e = hipGetLastError()) != hipSuccess) return e;
   // tau per row from the 2 CT partials of 128 units (centred: merged by
   // Chan's formula, no second pass over the stored scores)
-  if ((e = launch_tau(mom, a.in.tau_offset, tau, g.Tv, 2 * g.CT, g.N, 2, nullptr,
+  const bool dg = (d.flags & SRW_FLAG_DIAG) != 0;
+  float* token_diag = dg ? a.o.token_diag : nullptr;
+  float* unit_diag = dg ? a.o.unit_diag : nullptr;
+  const int tps = dg ? kTokPartDiag : 4;
+  const float exp_scale = -d.sharpness * 1.4426950408889634f;
+  if ((e = launch_tau(mom, a.in.tau_offset, tau, g.Tv, 2 * g.CT, g.N, 2, token_diag,
                       d.stats_mode == SRW_STATS_CENTERED ? kTauChan : kTauOnePass, a.stream, nullptr, 128)) !=
       hipSuccess)
     return e;
+  if (dg) {  // from the scores, before P replaces them
+    TiledDiagArgs da{};
+    da.S = P;
+    da.tau = tau;
+    da.part = reinterpret_cast<float*>(a.ws + l.diag);
+    da.unit_part = unit_diag ? reinterpret_cast<float2*>(a.ws + l.upart) : nullptr;
+    da.tok_sum = tok_sum;
+    da.token_diag = token_diag;
+    da.Tv = g.Tv;
+    da.N = g.N;
+    da.N64 = g.N64;
+    da.gp = a.gp;
+    da.exp_scale = exp_scale;
+    if ((e = tiled_diag(da, a.stream)) != hipSuccess) return e;
+    if (unit_diag && (e = launch_unit_diag(da.unit_part, (g.Tv + 31) / 32, g.N, unit_diag, a.gp, exp_scale, false,
+                                           a.stream)) != hipSuccess)
+      return e;
+  }
 
   if (tiled_sparse(d)) return tiled_sparse_rest(a, g, l);
 
@@ -1288,7 +1314,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   gp.RT = g.RT;
   gp.CT = g.CT;
   gp.gp = a.gp;
-  gp.exp_scale = -d.sharpness * 1.4426950408889634f;
+  gp.exp_scale = exp_scale;
   dominant_kernel_begin(a.stream);
   if (gp.G)
     hipLaunchKernelGGL((tiled_gate_kernel<false, true>), dim3(grid_rc), dim3(kGThreads), kGemmLds, a.stream, gp);
@@ -1316,7 +1342,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
   hipLaunchKernelGGL(tiled_tok_sum_kernel, dim3(static_cast<unsigned>((g.Tv + 63) / 64)), dim3(256), 0, a.stream,
-                     tok_part, tok_sum, g.Tv, 2 * g.CT);
+                     tok_part, tok_sum, g.Tv, 2 * g.CT, tps);
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
   FinalizeArgs f{};
@@ -1331,10 +1357,12 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   f.S = g.S;
   f.spc = g.spc;
   f.S_tok = 1;
-  f.tps = 4;
+  f.tps = tps;
   f.scale = d.scale;
+  f.tau = tau;
+  f.token_diag = token_diag;
   f.gp = a.gp;
-  f.exp_scale = -d.sharpness * 1.4426950408889634f;
+  f.exp_scale = exp_scale;
   return launch_finalize(f, a.stream);
 }
 
