@@ -56,7 +56,15 @@ EXPORTED_SYMBOLS = (
     "srw_workspace_size", "srw_forward", "srw_last_path",
     "srw_set_kernel_events", "srw_backward_workspace_size", "srw_backward",
     "srw_workspace_size_batch", "srw_forward_batch", "srw_forward_noalloc",
+    "srw_diag_summary", "srw_cast_bf16",
 )
+
+# srw_diag_out_t: the result tuple's per-token values and scalars (SRW_DSUM_*)
+DSUM_TOKEN = ("active_frac", "gate_max", "strong_frac", "boundary_frac", "z_mean_active")
+DSUM_SCALAR = ("score_lb", "score_std", "gate_sum", "active_n", "tau", "z_lt_075", "z_lt_030", "skew",
+               "active_std", "entropy", "int_sum", "kurt", "dead_penalty", "dead_count", "int_max", "int_cap")
+DSUM_WORKSPACE_BYTES = 64 << 10   # SRW_DSUM_WORKSPACE_BYTES
+MAX_CAST = 8                      # SRW_MAX_CAST
 
 
 class SrwDesc(ctypes.Structure):
@@ -91,6 +99,10 @@ class SrwCotangents(ctypes.Structure):
 class SrwGrads(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in (
         "dx", "dh", "demb", "dtau_offset", "dread", "dwrite", "dscale")]
+
+
+class SrwDiagOut(ctypes.Structure):
+    _fields_ = [("token", ctypes.c_void_p * len(DSUM_TOKEN)), ("scalar", ctypes.c_void_p * len(DSUM_SCALAR))]
 
 
 class SrwError(RuntimeError):
@@ -155,6 +167,14 @@ def load_library() -> ctypes.CDLL:
         lib.srw_backward.argtypes = [
             ctypes.POINTER(SrwDesc), ctypes.POINTER(SrwTensors), ctypes.POINTER(SrwCotangents),
             ctypes.POINTER(SrwGrads), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.srw_diag_summary.restype = ctypes.c_int
+        lib.srw_diag_summary.argtypes = [
+            ctypes.POINTER(SrwDesc), ctypes.POINTER(SrwOutputs), ctypes.POINTER(SrwDiagOut),
+            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.srw_cast_bf16.restype = ctypes.c_int
+        lib.srw_cast_bf16.argtypes = [
+            ctypes.c_int32, ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p),
+            ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p]
         got = lib.srw_abi_version()
         if got != ABI_VERSION:
             raise SrwLibraryError(f"libsrw_amd.so ABI {got} != binding ABI {ABI_VERSION}")

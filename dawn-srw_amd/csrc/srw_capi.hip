@@ -409,6 +409,34 @@ srw_status_t srw_backward(const srw_desc_t* d, const srw_tensors_t* in, const sr
   return e == hipSuccess ? SRW_OK : SRW_EHIP;
 }
 
+srw_status_t srw_diag_summary(const srw_desc_t* d, const srw_outputs_t* outs, const srw_diag_out_t* summary,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  const srw_status_t st = validate(d);
+  if (st != SRW_OK) return st;
+  if (!outs || !summary || d->T < 1) return SRW_EINVAL;
+  if (!outs->gate_sum || !outs->n_active || !outs->token_diag || !outs->unit_diag) return SRW_EINVAL;
+  if (!workspace || workspace_bytes < SRW_DSUM_WORKSPACE_BYTES) return SRW_EWORKSPACE;
+  if (reinterpret_cast<uintptr_t>(workspace) & 7) return SRW_EINVAL;
+  (void)hipGetLastError();
+  return srw::diag_summary(*d, *outs, *summary, static_cast<double*>(workspace), static_cast<hipStream_t>(stream)) ==
+                 hipSuccess
+             ? SRW_OK
+             : SRW_EHIP;
+}
+
+srw_status_t srw_cast_bf16(int32_t n, const float* const* src, void* const* dst, const int64_t* count,
+                           void* stream) {
+  if (n < 1 || n > SRW_MAX_CAST || !src || !dst || !count) return SRW_EINVAL;
+  uint16_t* out[SRW_MAX_CAST];
+  for (int32_t i = 0; i < n; ++i) {
+    if (count[i] < 0 || (count[i] > 0 && (!src[i] || !dst[i]))) return SRW_EINVAL;
+    if ((reinterpret_cast<uintptr_t>(src[i]) & 3) || (reinterpret_cast<uintptr_t>(dst[i]) & 1)) return SRW_EINVAL;
+    out[i] = static_cast<uint16_t*>(dst[i]);
+  }
+  (void)hipGetLastError();
+  return srw::cast_bf16(n, src, out, count, static_cast<hipStream_t>(stream)) == hipSuccess ? SRW_OK : SRW_EHIP;
+}
+
 const char* srw_last_path(void) { return g_last_path; }
 
 srw_status_t srw_set_kernel_events(void* start, void* stop) {

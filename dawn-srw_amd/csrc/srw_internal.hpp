@@ -147,6 +147,11 @@ struct TiledDiagArgs {
 };
 hipError_t tiled_diag(const TiledDiagArgs& a, hipStream_t s);
 
+// srw_diag_summary and srw_cast_bf16 (srw_diag.hip), arguments checked.
+hipError_t diag_summary(const srw_desc_t& d, const srw_outputs_t& o, const srw_diag_out_t& out, double* part,
+                        hipStream_t s);
+hipError_t cast_bf16(int n, const float* const* src, uint16_t* const* dst, const int64_t* count, hipStream_t s);
+
 // Tiled-GEMM kernels for wide layers (bf16), see srw_tiled.hip: P = gated
 // product materialised in HBM; d_model and d_route multiples of 64.
 bool tiled_supports(const srw_desc_t& d);

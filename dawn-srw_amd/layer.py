@@ -174,6 +174,48 @@ class SrwPlan:
                     path=self.path, workspace=self.workspace)
 
 
+def _stream_ptr(dev):
+    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+
+
+def cast_bf16(tensors, dev):
+    """The bf16 casts of a fused function's operands (v41:423-430), contiguous;
+    the float32 ones on ``dev`` share one launch."""
+    outs = list(tensors)
+    batch = [i for i, t in enumerate(outs)
+             if t.dtype == torch.float32 and t.device == dev and dev.type == "cuda" and t.numel()]
+    for a in range(0, len(batch), C.MAX_CAST):
+        idx = batch[a:a + C.MAX_CAST]
+        src = [outs[i].contiguous() for i in idx]
+        dst = [torch.empty(t.shape, dtype=torch.bfloat16, device=dev) for t in src]
+        n = len(idx)
+        with torch.cuda.device(dev):
+            C.check(C.load_library().srw_cast_bf16(
+                n, (ctypes.c_void_p * n)(*(t.data_ptr() for t in src)),
+                (ctypes.c_void_p * n)(*(t.data_ptr() for t in dst)),
+                (ctypes.c_int64 * n)(*(t.numel() for t in src)), _stream_ptr(dev)))
+        for i, t in zip(idx, dst):
+            outs[i] = t
+    return [t.to(torch.bfloat16).contiguous() for t in outs]
+
+
+def diag_summary(plan, lead):
+    """The fused functions' diagnostics (v41:588-635) from a ``diag=True``
+    plan's outputs: ({name: per-token [*lead, 1]}, {name: scalar})."""
+    dev, v401 = plan.device, plan._desc.gate == C.SRW_GATE_GELU_V401
+    names = C.DSUM_SCALAR[:10] if v401 else C.DSUM_SCALAR
+    tok = [torch.empty((*lead, 1), dtype=torch.float32, device=dev) for _ in C.DSUM_TOKEN]
+    sca = [torch.empty((), dtype=torch.float32, device=dev) for _ in names]
+    ws = torch.empty(C.DSUM_WORKSPACE_BYTES, dtype=torch.uint8, device=dev)
+    out = C.SrwDiagOut((ctypes.c_void_p * len(C.DSUM_TOKEN))(*(t.data_ptr() for t in tok)),
+                       (ctypes.c_void_p * len(C.DSUM_SCALAR))(*(t.data_ptr() for t in sca)))
+    with torch.cuda.device(dev):
+        C.check(plan._lib.srw_diag_summary(
+            ctypes.byref(plan._desc), ctypes.byref(plan._outs), ctypes.byref(out), _ptr(ws),
+            ctypes.c_size_t(C.DSUM_WORKSPACE_BYTES), _stream_ptr(dev)))
+    return dict(zip(C.DSUM_TOKEN, tok)), dict(zip(names, sca))
+
+
 class SrwBatchPlan:
     """Several bound calls enqueued together through ``srw_forward_batch``.
 

@@ -36,7 +36,7 @@ from __future__ import annotations
 
 import torch
 
-from .layer import GateConfig, srw_backward, srw_forward
+from .layer import GateConfig, SrwPlan, cast_bf16, diag_summary, srw_backward, srw_forward
 from . import _capi as C
 
 __all__ = ["make_sharded_srw", "make_sharded_srw_paired", "make_sharded_srw_v401",
@@ -134,6 +134,38 @@ _NAMES = ("out", "active_frac", "gate_max", "score_lb", "score_std", "gate_sum_m
           "kurt", "dead_penalty", "dead_count", "int_max", "int_cap_frac")
 
 
+def _call_operands(x, h, emb, tau_offset, read, write, routes):
+    """The bf16 operands (v41:423-430): (x [T, D], h [T, R, dr], the h to call
+    with, emb, tau [T, R] float32, read, write).  Where the caller's h is x
+    itself (score = x.E^T, one route) the call gets the one tensor, which lets
+    the kernels hold a single operand in registers."""
+    B, S, D = x.shape
+    same = h is x and routes == 1
+    ts = [x.reshape(B * S, D), emb, read, write]
+    if not same:
+        ts.append(h.reshape(B * S, routes, h.shape[-1]))
+    xb, eb, rdb, wb, *rest = cast_bf16(ts, x.device)
+    hb = xb.view(B * S, 1, D) if same else rest[0]
+    tau = tau_offset.reshape(B * S, routes).to(torch.float32).contiguous()
+    return xb, hb, xb if same else hb, eb, tau, rdb, wb
+
+
+def _fused_diag(plan, N, B, S, R, dead_threshold, v401):
+    """The diagnostics after out, from the kernels' columns in two launches;
+    an empty call's go through the torch form (its means and maxima of
+    nothing are torch's)."""
+    if B * S == 0:
+        res = plan.results()
+        return _diag_tuple_v401(res, N, B, S, R) if v401 else _diag_tuple(res, N, B, S, R, dead_threshold)
+    t, c = diag_summary(plan, (B, S))
+    head = (t["active_frac"], t["gate_max"], c["score_lb"], c["score_std"], c["gate_sum"], c["active_n"],
+            t["strong_frac"], t["boundary_frac"], t["z_mean_active"], c["tau"], c["z_lt_075"], c["z_lt_030"],
+            c["skew"], c["active_std"], c["entropy"])
+    if v401:
+        return head
+    return head + (c["int_sum"], c["kurt"], c["dead_penalty"], c["dead_count"], c["int_max"], c["int_cap"])
+
+
 class _FusedSrw(torch.autograd.Function):
     """fused_gate_srw(_paired) as one autograd node: the forward runs
     srw_forward (bf16, one-pass statistics, diagnostics), the backward runs
@@ -148,19 +180,14 @@ class _FusedSrw(torch.autograd.Function):
     def forward(ctx, x, h, emb, tau_offset, read, write, routes, consts, cs):
         B, S, D = x.shape
         N = emb.shape[0]
-        bf = torch.bfloat16
-        xb = x.reshape(B * S, D).to(bf).contiguous()
-        hb = h.reshape(B * S, routes, h.shape[-1]).to(bf).contiguous()
-        tau = tau_offset.reshape(B * S, routes).to(torch.float32).contiguous()
-        eb, rdb, wb = (t.to(bf).contiguous() for t in (emb, read, write))
-        # the caller's h is x itself (score = x.E^T, one route): pass the one
-        # tensor, which lets the kernels hold a single operand in registers
-        h_call = xb if (h is x and routes == 1) else hb
-        res = srw_forward(xb, h_call, eb, tau, rdb, wb, stats="onepass", consts=consts,
-                          chunk_size=cs, diag=True, want_mask=False)
+        xb, hb, h_call, eb, tau, rdb, wb = _call_operands(x, h, emb, tau_offset, read, write, routes)
+        plan = SrwPlan(xb, h_call, eb, tau, rdb, wb, stats="onepass", consts=consts, chunk_size=cs, diag=True,
+                       want_mask=False)
+        plan.launch()
+        res = plan.results()
         shape = (B, S, D) if routes == 1 else (B, S, 2, D)
         out = res["out"].reshape(shape).to(torch.float32)
-        outs = (out,) + _diag_tuple(res, N, B, S, routes, consts.dead_threshold)
+        outs = (out,) + _fused_diag(plan, N, B, S, routes, consts.dead_threshold, False)
         # the forward's den and unit statistics: the backward takes them
         # instead of recomputing them from the scores
         ctx.save_for_backward(xb, hb, eb, tau, rdb, wb, res["out"], res["den"], res["unit_diag"])
@@ -284,17 +311,14 @@ class _FusedSrwV401(torch.autograd.Function):
     def forward(ctx, x, h, emb, tau_offset, read, write, routes, cs):
         B, S, D = x.shape
         N = emb.shape[0]
-        bf = torch.bfloat16
-        xb = x.reshape(B * S, D).to(bf).contiguous()                       # v401:238-242
-        hb = h.reshape(B * S, routes, h.shape[-1]).to(bf).contiguous()
-        tau = tau_offset.reshape(B * S, routes).to(torch.float32).contiguous()
-        eb, rdb, wb = (t.to(bf).contiguous() for t in (emb, read, write))
-        h_call = xb if (h is x and routes == 1) else hb
-        res = srw_forward(xb, h_call, eb, tau, rdb, wb, gate="gelu_v401", stats="onepass",
-                          chunk_size=cs, diag=True, want_mask=False)
+        xb, hb, h_call, eb, tau, rdb, wb = _call_operands(x, h, emb, tau_offset, read, write, routes)  # v401:238-242
+        plan = SrwPlan(xb, h_call, eb, tau, rdb, wb, gate="gelu_v401", stats="onepass", chunk_size=cs, diag=True,
+                       want_mask=False)
+        plan.launch()
+        res = plan.results()
         shape = (B, S, D) if routes == 1 else (B, S, 2, D)
         out = res["out"].reshape(shape).to(torch.float32)
-        outs = (out,) + _diag_tuple_v401(res, N, B, S, routes)
+        outs = (out,) + _fused_diag(plan, N, B, S, routes, 0.0, True)
         ctx.save_for_backward(xb, hb, eb, tau, rdb, wb, res["out"], res["den"], res["unit_diag"])
         ctx.meta = (routes, tuple(t.shape for t in (x, h, emb, tau_offset, read, write)),
                     tuple(t.dtype for t in (x, h, emb, tau_offset, read, write)))

@@ -327,6 +327,55 @@ srw_status_t srw_backward(const srw_desc_t* desc, const srw_tensors_t* in,
                           const srw_cotangents_t* cot, const srw_grads_t* grads,
                           void* workspace, size_t workspace_bytes, void* stream);
 
+/* The diagnostics of the fused functions' result tuples (v41:588-635 single,
+ * :862-907 paired; v4.0.1: v401:343-367, :525-553) from a SRW_FLAG_DIAG call's
+ * outputs.  Per-token values [T], averaged over the routes where n_routes ==
+ * 2; scalars [1], over every (token, route) row or every unit. */
+enum {
+  SRW_DSUM_ACTIVE_FRAC = 0, /* n_active / N */
+  SRW_DSUM_GATE_MAX,
+  SRW_DSUM_STRONG_FRAC,
+  SRW_DSUM_BOUNDARY_FRAC,
+  SRW_DSUM_Z_MEAN_ACTIVE,   /* gate_sum / n_active (v4.0.1: sum z+ / n_active) */
+  SRW_DSUM_TOKEN_COUNT
+};
+enum {
+  SRW_DSUM_SCORE_LB = 0,
+  SRW_DSUM_SCORE_STD,
+  SRW_DSUM_GATE_SUM,
+  SRW_DSUM_ACTIVE_N,
+  SRW_DSUM_TAU,
+  SRW_DSUM_Z_LT_075,
+  SRW_DSUM_Z_LT_030,
+  SRW_DSUM_SKEW,
+  SRW_DSUM_ACTIVE_STD,
+  SRW_DSUM_ENTROPY,
+  SRW_DSUM_INT_SUM,         /* v4.1 from here on */
+  SRW_DSUM_KURT,
+  SRW_DSUM_DEAD_PENALTY,
+  SRW_DSUM_DEAD_COUNT,
+  SRW_DSUM_INT_MAX,
+  SRW_DSUM_INT_CAP,
+  SRW_DSUM_SCALAR_COUNT
+};
+typedef struct srw_diag_out {
+  float* token[SRW_DSUM_TOKEN_COUNT];   /* [T] each, or NULL */
+  float* scalar[SRW_DSUM_SCALAR_COUNT]; /* [1] each, or NULL */
+} srw_diag_out_t;
+
+/* Two launches; sums in double, in a fixed order.  desc as the forward
+ * call's (T, n_routes, n_units, gate, dead_threshold are read; T > 0);
+ * outs->gate_sum, n_active, token_diag and unit_diag as that call wrote them.
+ * workspace: SRW_DSUM_WORKSPACE_BYTES of device memory. */
+#define SRW_DSUM_WORKSPACE_BYTES ((size_t)64 << 10)
+srw_status_t srw_diag_summary(const srw_desc_t* desc, const srw_outputs_t* outs, const srw_diag_out_t* summary,
+                              void* workspace, size_t workspace_bytes, void* stream);
+
+/* dst[i][k] = bf16(src[i][k]) for k < count[i], i < n: the casts of a fused
+ * function's operands (v41:423-430) in one launch.  1 <= n <= SRW_MAX_CAST. */
+#define SRW_MAX_CAST 8
+srw_status_t srw_cast_bf16(int32_t n, const float* const* src, void* const* dst, const int64_t* count, void* stream);
+
 /* Name of the kernel family the last srw_forward on this thread used
  * ("generic", "mfma_bf16", "mfma_ss_bf16", ...), for tests and benchmarks. */
 const char* srw_last_path(void);
