@@ -56,7 +56,7 @@ EXPORTED_SYMBOLS = (
     "srw_workspace_size", "srw_forward", "srw_last_path",
     "srw_set_kernel_events", "srw_backward_workspace_size", "srw_backward",
     "srw_workspace_size_batch", "srw_forward_batch", "srw_forward_noalloc",
-    "srw_diag_summary", "srw_cast_bf16",
+    "srw_diag_summary", "srw_cast_bf16", "srw_dawn_decode_step",
 )
 
 # srw_diag_out_t: the result tuple's per-token values and scalars (SRW_DSUM_*)
@@ -103,6 +103,27 @@ class SrwGrads(ctypes.Structure):
 
 class SrwDiagOut(ctypes.Structure):
     _fields_ = [("token", ctypes.c_void_p * len(DSUM_TOKEN)), ("scalar", ctypes.c_void_p * len(DSUM_SCALAR))]
+
+
+class SrwDawnLayer(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in (
+        "norm1_scale", "norm1_bias", "norm2_scale", "norm2_bias", "expand_o")]
+
+
+class SrwDawnStep(ctypes.Structure):
+    _fields_ = (
+        [(n, ctypes.c_int64) for n in ("B", "d_model", "d_route", "max_seq", "pos")]
+        + [(n, ctypes.c_int32) for n in ("n_layers", "n_heads", "qkv_cached", "know_cached")]
+        + [("layers", ctypes.POINTER(SrwDawnLayer))]
+        + [(n, ctypes.c_void_p) for n in (
+            "proj_attn_w", "proj_attn_b", "tau_attn_w", "tau_attn_b", "proj_know_w", "proj_know_b",
+            "tau_know_w", "tau_know_b", "norm_scale", "norm_bias", "qk_scale", "v_scale", "know_scale",
+            "x", "x_alt", "attn", "cache_k", "cache_v", "normed")]
+        + [("descs", ctypes.POINTER(SrwDesc)), ("tensors", ctypes.POINTER(SrwTensors)),
+           ("outs", ctypes.POINTER(SrwOutputs)),
+           ("ws_qkv", ctypes.c_void_p), ("ws_qkv_bytes", ctypes.c_size_t),
+           ("ws_know", ctypes.c_void_p), ("ws_know_bytes", ctypes.c_size_t),
+           ("path_qkv", ctypes.POINTER(ctypes.c_char_p))])
 
 
 class SrwError(RuntimeError):
@@ -175,6 +196,8 @@ def load_library() -> ctypes.CDLL:
         lib.srw_cast_bf16.argtypes = [
             ctypes.c_int32, ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p),
             ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p]
+        lib.srw_dawn_decode_step.restype = ctypes.c_int
+        lib.srw_dawn_decode_step.argtypes = [ctypes.POINTER(SrwDawnStep), ctypes.c_void_p]
         got = lib.srw_abi_version()
         if got != ABI_VERSION:
             raise SrwLibraryError(f"libsrw_amd.so ABI {got} != binding ABI {ABI_VERSION}")

@@ -424,6 +424,46 @@ srw_status_t srw_diag_summary(const srw_desc_t* d, const srw_outputs_t* outs, co
              : SRW_EHIP;
 }
 
+srw_status_t srw_dawn_decode_step(const srw_dawn_step_t* s, void* stream) {
+  if (!s || !s->layers || !s->descs || !s->tensors || !s->outs || s->n_layers < 1) return SRW_EINVAL;
+  if (s->pos < 0 || s->pos >= s->max_seq) return SRW_EINVAL;
+  if (!srw::dawn_step_supports(*s)) return SRW_EUNSUPPORTED;
+  for (const void* q : {static_cast<const void*>(s->proj_attn_w), static_cast<const void*>(s->proj_attn_b),
+                        static_cast<const void*>(s->tau_attn_w), static_cast<const void*>(s->tau_attn_b),
+                        static_cast<const void*>(s->proj_know_w), static_cast<const void*>(s->proj_know_b),
+                        static_cast<const void*>(s->tau_know_w), static_cast<const void*>(s->tau_know_b),
+                        static_cast<const void*>(s->qk_scale), static_cast<const void*>(s->v_scale),
+                        static_cast<const void*>(s->know_scale)})
+    if (!q) return SRW_EINVAL;
+  // rows are read and written in 16-byte pieces
+  auto wide = [](const void* q) { return q && !(reinterpret_cast<uintptr_t>(q) & 15); };
+  if (!wide(s->x) || !wide(s->x_alt) || !wide(s->attn) || !wide(s->cache_k) || !wide(s->cache_v) ||
+      !wide(s->normed) || !wide(s->norm_scale) || !wide(s->norm_bias))
+    return SRW_EINVAL;
+  for (int32_t i = 0; i < s->n_layers; ++i) {
+    const srw_dawn_layer_t& l = s->layers[i];
+    if (!wide(l.norm1_scale) || !wide(l.norm1_bias) || !wide(l.norm2_scale) || !wide(l.norm2_bias) || !l.expand_o)
+      return SRW_EINVAL;
+  }
+  for (int32_t i = 0; i < 3; ++i) {
+    const srw_desc_t& d = s->descs[i];
+    if (validate(&d) != SRW_OK || d.dtype != SRW_BF16 || d.T != s->B || d.d_model != s->d_model ||
+        d.d_route != s->d_route || d.n_routes != (i == 0 ? 2 : 1))
+      return SRW_EINVAL;
+    if (!wide(s->tensors[i].x) || !wide(s->tensors[i].h) || !s->tensors[i].tau_offset || !wide(s->outs[i].out))
+      return SRW_EINVAL;
+  }
+  // the SRW calls inside must pass before anything is launched
+  size_t need = 0;
+  srw_status_t st = srw_workspace_size_batch(2, s->descs, &need);
+  if (st != SRW_OK) return st;
+  if (need > 0 && (!s->ws_qkv || s->ws_qkv_bytes < need)) return SRW_EWORKSPACE;
+  if ((st = srw_workspace_size(&s->descs[2], &need)) != SRW_OK) return st;
+  if (need > 0 && (!s->ws_know || s->ws_know_bytes < need)) return SRW_EWORKSPACE;
+  (void)hipGetLastError();
+  return srw::dawn_decode_step(*s, static_cast<hipStream_t>(stream)) == hipSuccess ? SRW_OK : SRW_EHIP;
+}
+
 srw_status_t srw_cast_bf16(int32_t n, const float* const* src, void* const* dst, const int64_t* count,
                            void* stream) {
   if (n < 1 || n > SRW_MAX_CAST || !src || !dst || !count) return SRW_EINVAL;

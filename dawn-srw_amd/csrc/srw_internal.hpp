@@ -152,6 +152,10 @@ hipError_t diag_summary(const srw_desc_t& d, const srw_outputs_t& o, const srw_d
                         hipStream_t s);
 hipError_t cast_bf16(int n, const float* const* src, uint16_t* const* dst, const int64_t* count, hipStream_t s);
 
+// srw_dawn_decode_step (srw_model.hip), arguments checked.
+bool dawn_step_supports(const srw_dawn_step_t& s);
+hipError_t dawn_decode_step(const srw_dawn_step_t& s, hipStream_t st);
+
 // Tiled-GEMM kernels for wide layers (bf16), see srw_tiled.hip: P = gated
 // product materialised in HBM; d_model and d_route multiples of 64.
 bool tiled_supports(const srw_desc_t& d);

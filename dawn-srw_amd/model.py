@@ -19,12 +19,14 @@ tree names (``params['neuron_pool']['know_emb']``,
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
 
+from . import _capi as C
 from .layer import GateConfig, SrwBatchPlan, SrwPlan
 from .srw import chunk_plan
 
@@ -296,6 +298,64 @@ class DawnModel:
         x = self._ln(x, self.p["norm"])
         return (x @ self.p["token_emb"]["embedding"].T).reshape(B, S, -1), cK, cV, S
 
+    def _decode_native(self, x, cache_K, cache_V, cache_len):
+        """The layers of a decode step in one library call
+        (``srw_dawn_decode_step``), from the embedded rows x [B, D] to the
+        final LayerNorm's; None where the call does not apply: more rows than
+        one batch of decode-sized calls, widths the kernels do not take, or
+        caches and parameters that are not contiguous float32 on the device."""
+        cfg, dev = self.cfg, self.device
+        B, D = x.shape
+        H, dr, L = cfg.n_heads, cfg.d_route, cfg.n_layers
+        if not (1 <= B and 2 * B <= 128 and D in (128, 384) and D == 64 * H and dr % 16 == 0 and cache_len >= 0):
+            return None
+        rt, pool = self.p["router"], self.p["neuron_pool"]
+        par = {"proj_attn_w": (rt["proj_attn"]["kernel"], (D, 3 * dr)), "proj_attn_b": (rt["proj_attn"]["bias"], (3 * dr,)),
+               "tau_attn_w": (rt["tau_attn"]["kernel"], (D, 3)), "tau_attn_b": (rt["tau_attn"]["bias"], (3,)),
+               "proj_know_w": (rt["proj_know"]["kernel"], (D, dr)), "proj_know_b": (rt["proj_know"]["bias"], (dr,)),
+               "tau_know_w": (rt["tau_know"]["kernel"], (D, 1)), "tau_know_b": (rt["tau_know"]["bias"], (1,)),
+               "norm_scale": (self.p["norm"]["scale"], (D,)), "norm_bias": (self.p["norm"]["bias"], (D,)),
+               "qk_scale": (self.scale["qk"], (1,)), "v_scale": (self.scale["v"], (1,)),
+               "know_scale": (self.scale["know"], (1,)),
+               "cache_k": (cache_K, (L, B, H, cfg.max_seq_len, 64)), "cache_v": (cache_V, (L, B, H, cfg.max_seq_len, 64))}
+        layers = (C.SrwDawnLayer * L)()
+        checked = list(par.values())
+        for i in range(L):
+            bp = self.p[f"block_{i}"]
+            for f, t, shape in (("norm1_scale", bp["norm1"]["scale"], (D,)), ("norm1_bias", bp["norm1"]["bias"], (D,)),
+                                ("norm2_scale", bp["norm2"]["scale"], (D,)), ("norm2_bias", bp["norm2"]["bias"], (D,)),
+                                ("expand_o", bp["attn"]["expand_O"]["kernel"], (D, D))):
+                checked.append((t, shape))
+                setattr(layers[i], f, t.data_ptr())
+        for t, shape in checked:
+            if (t.dtype != F32 or t.device != x.device or t.shape != shape or not t.is_contiguous()
+                    or t.data_ptr() % (16 if len(shape) == 5 or shape == (D,) else 4)):
+                return None
+        qkv, know = self._qkv_batch(B, "centered"), self._pool("know", B, 1, "centered")
+        x = x.contiguous()
+        x_alt, attn, normed = (torch.empty_like(x) for _ in range(3))
+        plans = [qkv.calls[0].plan, qkv.calls[1].plan, know.plan]
+        path = (ctypes.c_char_p * 1)()
+        s = C.SrwDawnStep(B=B, path_qkv=path, d_model=D, d_route=dr, max_seq=cfg.max_seq_len, pos=int(cache_len), n_layers=L,
+                          n_heads=H, qkv_cached=qkv.launches > 0, know_cached=know.launches > 0, layers=layers,
+                          x=x.data_ptr(), x_alt=x_alt.data_ptr(), attn=attn.data_ptr(), normed=normed.data_ptr(),
+                          descs=(C.SrwDesc * 3)(*(p._desc for p in plans)),
+                          tensors=(C.SrwTensors * 3)(*(p._tens for p in plans)),
+                          outs=(C.SrwOutputs * 3)(*(p._outs for p in plans)),
+                          ws_qkv=qkv.plan.workspace.data_ptr(), ws_qkv_bytes=qkv.plan.ws_bytes,
+                          ws_know=know.plan.workspace.data_ptr(), ws_know_bytes=know.plan.ws_bytes,
+                          **{k: t.data_ptr() for k, (t, _) in par.items()})
+        with torch.cuda.device(dev):
+            C.check(C.load_library().srw_dawn_decode_step(
+                ctypes.byref(s), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)))
+        qkv.launches += L
+        know.launches += L
+        qkv.plan.path = path[0].decode()
+        for p in qkv.plan.plans:
+            p.path = qkv.plan.path
+        know.plan.path = C.last_path()
+        return normed
+
     @torch.no_grad()
     def decode_step(self, token_id, cache_K, cache_V, cache_len: int):
         """One token per sequence with the KV cache (v41:1914-1957):
@@ -309,6 +369,9 @@ class DawnModel:
         D, H = cfg.d_model, cfg.n_heads
         dh = D // H
         x = self._embed(ids, pos0=cache_len).reshape(B, D)
+        n = self._decode_native(x, cache_K, cache_V, cache_len)
+        if n is not None:
+            return n @ self.p["token_emb"]["embedding"].T, cache_K, cache_V, cache_len + 1
         scale = math.sqrt(dh)
         for i in range(cfg.n_layers):
             bp = self.p[f"block_{i}"]

@@ -371,6 +371,45 @@ typedef struct srw_diag_out {
 srw_status_t srw_diag_summary(const srw_desc_t* desc, const srw_outputs_t* outs, const srw_diag_out_t* summary,
                               void* workspace, size_t workspace_bytes, void* stream);
 
+/* One KV-cache decode step of the DAWN model (v41:1772-1828, 1914-1957) from
+ * the embedded rows to the final LayerNorm: per layer LayerNorm + router, the
+ * QK (paired) and V calls as srw_forward_batch, the caches' new rows and the
+ * attention over them, expand_O + residual, LayerNorm + router, the Know
+ * call.  Parameters float32 on the device; host arrays where noted.  The
+ * router's products and the normalised rows are written into the calls'
+ * tensors (tensors[i].x, h, tau_offset are the caller's buffers). */
+typedef struct srw_dawn_layer {
+  const float *norm1_scale, *norm1_bias, *norm2_scale, *norm2_bias; /* [d_model] */
+  const float* expand_o;                                            /* [d_model, d_model] */
+} srw_dawn_layer_t;
+typedef struct srw_dawn_step {
+  int64_t B, d_model, d_route, max_seq;
+  int64_t pos;                  /* positions in the caches; the new rows go there (pos < max_seq) */
+  int32_t n_layers, n_heads;
+  int32_t qkv_cached, know_cached; /* the workspaces hold this pool's packed rows (SRW_FLAG_POOL_CACHED) */
+  const srw_dawn_layer_t* layers;  /* host, [n_layers] */
+  const float *proj_attn_w, *proj_attn_b; /* [d_model, 3 d_route], [3 d_route] */
+  const float *tau_attn_w, *tau_attn_b;   /* [d_model, 3], [3] */
+  const float *proj_know_w, *proj_know_b; /* [d_model, d_route], [d_route] */
+  const float *tau_know_w, *tau_know_b;   /* [d_model, 1], [1] */
+  const float *norm_scale, *norm_bias;    /* the final LayerNorm */
+  const float *qk_scale, *v_scale, *know_scale; /* [1] */
+  float *x, *x_alt, *attn;      /* [B, d_model]: the embedded rows, overwritten; scratch; scratch */
+  float *cache_k, *cache_v;     /* [n_layers, B, n_heads, max_seq, 64] */
+  float* normed;                /* [B, d_model]: the result */
+  const srw_desc_t* descs;      /* host, [3]: QK (n_routes 2), V, Know, T = B */
+  const srw_tensors_t* tensors; /* host, [3] */
+  const srw_outputs_t* outs;    /* host, [3] */
+  void* ws_qkv;                 /* srw_workspace_size_batch(2, descs) bytes */
+  size_t ws_qkv_bytes;
+  void* ws_know;                /* srw_workspace_size(&descs[2]) bytes */
+  size_t ws_know_bytes;
+  const char** path_qkv;        /* host: srw_last_path() after the QK and V calls; or NULL */
+} srw_dawn_step_t;
+/* d_model 128 or 384, heads of 64, d_route a multiple of 16; else
+ * SRW_EUNSUPPORTED with nothing launched. */
+srw_status_t srw_dawn_decode_step(const srw_dawn_step_t* step, void* stream);
+
 /* dst[i][k] = bf16(src[i][k]) for k < count[i], i < n: the casts of a fused
  * function's operands (v41:423-430) in one launch.  1 <= n <= SRW_MAX_CAST. */
 #define SRW_MAX_CAST 8
