@@ -61,6 +61,8 @@ __device__ inline int gswz(int u) { return (u & 7) ^ ((u >> 3) & 1); }
 struct Opnd {
   const char* base;  // byte address of memory row row0 / div, k = 0 (uniform)
   uint32_t off[8];   // per-lane byte offsets from base: row and swizzled piece
+  __device__ const char* block(int64_t kk) const { return base + kk * 2; }
+  __device__ const char* src(const char* blk, int q) const { return blk + off[q]; }
 };
 
 __device__ inline Opnd make_opnd(const uint16_t* p, int64_t ld, int64_t row0, int64_t rows, int div, int wave,
@@ -79,6 +81,64 @@ __device__ inline Opnd make_opnd(const uint16_t* p, int64_t ld, int64_t row0, in
   return o;
 }
 
+// An operand whose rows are k -- element (k, c) at p[k * ld + c], tile columns
+// contiguous in memory (P, d(xr) and ds [rows, N64] as the gradient products'
+// K = rows operands, x, h, R, E as their right-hand sides) -- staged as it
+// lies: 64 k-rows of C columns, read back transposed (ds_read_b64_tr_b16: 16
+// lanes exchange a 4 x 16 block, so that a lane gets four k of its column).
+// A row's 64-byte chunks (32 columns, one MFMA operand's) are XOR-swizzled so
+// that the four k-rows of a read lie in different banks: chunk c of row r at
+// c ^ (r & 3) of 512-byte rows, c ^ (r >> 1 & 1) of 384-byte ones (which
+// alternate between the halves of the banks by themselves).
+// Rows past the last k must be there and zero: in arrays of the workspace they
+// are; of a caller's array the last, partial block is read from a zero-padded
+// copy (`tail`, the same row length).
+struct KRows {
+  const uint16_t* p;
+  int64_t ld;            // elements per row
+  const uint16_t* tail;  // block from row kt on, or null
+  int64_t kt;
+};
+template <int C>  // 256 or 192 columns
+struct OpndT {
+  static constexpr int L = C / 32;        // 16-byte loads per lane and block
+  static constexpr int PPR = C / 8;       // 16-byte pieces per row
+  static constexpr int LV = C == 256 ? 1 : L;  // 512-byte rows: a lane's loads are eight rows apart, one piece
+  __host__ __device__ static constexpr int swz(int r) { return C == 256 ? r & 3 : (r >> 1) & 1; }
+  const char *base, *tail;  // byte address of row 0 (of the tail's first row), column c0 (uniform)
+  int64_t ldb, kt;          // bytes per k-row; first k of the tail block
+  uint32_t off[LV];
+  // the block whose first k is kk, and byte of its load q
+  __device__ const char* block(int64_t kk) const { return kk >= kt ? tail : base + kk * ldb; }
+  __device__ const char* src(const char* blk, int q) const {
+    return C == 256 ? blk + 8 * q * ldb + off[0] : blk + off[q % LV];
+  }
+};
+template <int C>
+__device__ inline OpndT<C> make_opnd_t(const KRows& k, int64_t c0, int wave, int lane) {
+  OpndT<C> o;
+  o.base = reinterpret_cast<const char*>(k.p + c0);
+  o.tail = reinterpret_cast<const char*>(k.tail + c0);
+  o.kt = k.tail ? k.kt : INT64_MAX;
+  o.ldb = k.ld * 2;
+#pragma unroll
+  for (int q = 0; q < OpndT<C>::LV; ++q) {
+    const int piece = 64 * (4 * q + wave) + lane;
+    const int r = piece / OpndT<C>::PPR, w = piece % OpndT<C>::PPR;
+    int64_t col = 8 * (4 * ((w >> 2) ^ OpndT<C>::swz(r)) + (w & 3));
+    col = c0 + col + 8 <= k.ld ? col : k.ld - 8 - c0;  // columns past the array: never stored
+    o.off[q] = static_cast<uint32_t>(r * o.ldb + col * 2);
+  }
+  return o;
+}
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+__device__ inline u32x4_t read_tr(const char* at, int step) {  // two reads four k-rows (step bytes) apart
+  typedef __attribute__((address_space(3))) i16x4_t* ptr;
+  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+  const u32x2_t a = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(at)));
+  const u32x2_t b = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(at + step)));
+  return u32x4_t{a[0], a[1], b[0], b[1]};
+}
 // acc[i][j] += A-tile rows (128 wa + 32 i ..) . B-tile rows (128 wb + 32 j ..)^T over
 // k in [k0, k0 + 64 nk), wave = 2 wa + wb.  hook(kb, stage) runs once block kb
 // has landed in LDS, before any wave reads it (all threads call it).
@@ -169,6 +229,101 @@ __device__ inline void gemm_loop(f32x16_t (&acc)[4][NBF], const Opnd& A, const O
   }
   wait_vm0();
   __syncthreads();  // the trailing reloads have landed before LDS is reused
+}
+
+// The same products with the B operand's rows k (OpndT), and A's as they are
+// (Opnd) or k as well: tiles of 64-k blocks, the barrier and the fragment order
+// as above, but the blocks come through registers -- loaded two blocks ahead,
+// written into the stage that k-step 3 frees.  (With direct global->LDS loads
+// in flight the compiler drains them, vmcnt(0), before every transposed read:
+// the Know pool's five products 1 050 us instead of 468.)
+template <int NBF, class OA>
+__device__ inline void gemm_loop_k(f32x16_t (&acc)[4][NBF], const OA& A, const OpndT<64 * NBF>& B, int64_t k0, int nk,
+                                   char* lds, int wave, int lane) {
+  constexpr bool KA = !std::is_same<OA, Opnd>::value;
+  constexpr int NB = 64 * NBF, NL = 8 + NB / 32, NQ = 4 * NBF, NF = 4 + NBF;
+  constexpr int STAGE = kOpBytes + NB * kGK * 2;
+  const int wa = wave >> 1, wb = wave & 1;
+  const int u = lane & 31, h = lane >> 5;
+  int le[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) le[m] = (u >> 3) * 1024 + (u & 7) * 128 + (((2 * m + h) ^ gswz(u)) * 16);
+  // the lane's byte of k-row 8 (lane / 32) + lane % 16 / 4 in MFMA operand g's chunk
+  int ta[4], tb[NBF];
+  {
+    const int r = 8 * h + ((lane >> 2) & 3), in = (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) ta[g] = r * 512 + ((4 * wa + g) ^ OpndT<256>::swz(r)) * 64 + in;
+#pragma unroll
+    for (int g = 0; g < NBF; ++g) tb[g] = kOpBytes + r * NB * 2 + ((NBF * wb + g) ^ OpndT<NB>::swz(r)) * 64 + in;
+  }
+  u32x4_t reg[NL];
+  // block b (past the last: the last one again, in bounds, never used)
+  auto first = [&](int b) { return k0 + static_cast<int64_t>(b < nk ? b : nk - 1) * kGK; };
+  auto load = [&](int q, const char* pa, const char* pb) {
+    reg[q] = *reinterpret_cast<const u32x4_t*>(q < 8 ? A.src(pa, q) : B.src(pb, q - 8));
+  };
+  auto put = [&](int q, char* stage) {
+    char* at = q < 8 ? stage + q * kGroupBytes : stage + kOpBytes + (q - 8) * kGroupBytes;
+    *reinterpret_cast<u32x4_t*>(at + wave * 1024 + lane * 16) = reg[q];
+  };
+  auto frag = [&](const char* stage, int g, int m) {
+    if (g < 4) {
+      if constexpr (KA) return read_tr(stage + ta[g < 4 ? g : 0] + 16 * m * 512, 4 * 512);
+      else return *reinterpret_cast<const u32x4_t*>(stage + (4 * wa + g) * kGroupBytes + le[m]);
+    } else {
+      return read_tr(stage + tb[g < 4 ? 0 : g - 4] + 16 * m * NB * 2, 4 * NB * 2);
+    }
+  };
+  auto order = [](int r) { return r == 0 ? 0 : (r <= NBF ? 3 + r : r - NBF); };
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    const char *pa = A.block(first(b)), *pb = B.block(first(b));
+#pragma unroll
+    for (int q = 0; q < NL; ++q) load(q, pa, pb);
+    if (b == 2) break;
+#pragma unroll
+    for (int q = 0; q < NL; ++q) put(q, lds + b * STAGE);
+  }
+  barrier_lds();
+  u32x4_t f[2][NF];
+#pragma unroll
+  for (int g = 0; g < NF; ++g) f[0][g] = frag(lds, g, 0);
+  for (int kb = 0; kb < nk; ++kb) {
+    char* st = lds + (kb & 1) * STAGE;
+    char* nxt = lds + ((kb & 1) ^ 1) * STAGE;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int cb = m & 1;
+      const char *pa = nullptr, *pb = nullptr;
+      if (m == 3) {
+        pa = A.block(first(kb + 3));
+        pb = B.block(first(kb + 3));
+        __builtin_amdgcn_sched_barrier(0);
+        barrier_lds();  // block kb + 1 is in LDS; nobody reads block kb's stage any more
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        acc[q / NBF][q % NBF] = mfma(f[cb][q / NBF], f[cb][4 + q % NBF], acc[q / NBF][q % NBF]);
+#pragma unroll
+        for (int r = 0; r < NF; ++r) {
+          if (r * NQ / NF == q) {
+            const int g = order(r);
+            f[cb ^ 1][g] = m < 3 ? frag(st, g, m + 1) : frag(nxt, g, 0);
+          }
+        }
+        if (m == 3) {
+#pragma unroll
+          for (int L = q * NL / NQ; L < (q + 1) * NL / NQ; ++L) {
+            put(L, st);
+            load(L, pa, pb);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __syncthreads();
 }
 
 // LDS of a gemm_loop<NBF> workgroup: two stages of the A and B tiles
@@ -855,6 +1010,8 @@ __global__ __launch_bounds__(kSpThreads, 1) void sp_gather_kernel(SpGatherParams
 struct TWriteParams {
   const uint16_t* P;   // [Tv, N64]
   const uint16_t* wt;  // [D, N64]
+  KRows ka, kb;        // the backward's products: operands whose rows are k, in place of wt and (a_rows) P
+  int a_rows;
   float* out_part;     // [S][Tv][D]
   int64_t Tv, N, N64, D, cs;
   int nc, spc, S, RT, DT;
@@ -879,7 +1036,8 @@ __device__ inline void mask_units(char* tile, int64_t kbase, int64_t lo, int64_t
 // MAYROUND: p.round_out is honoured (the backward's products); without it
 // the kernel has no rounding code (the forward's write GEMM: its register
 // allocation spilled with the rounded form compiled in beside the plain one).
-template <int NBF, bool MAYROUND>
+// KA, KB: the operand's rows are k (N of them).
+template <int NBF, bool MAYROUND, bool KA = false, bool KB = false>
 __device__ __attribute__((always_inline)) inline void write_body(const TWriteParams& p, const int bid) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -898,8 +1056,14 @@ __device__ __attribute__((always_inline)) inline void write_body(const TWritePar
   const int64_t b_lo = lo / kGK, b_hi = (hi + kGK - 1) / kGK, nb = b_hi - b_lo;
   const int64_t kb0 = b_lo + nb * sub / p.spc, kb1 = b_lo + nb * (sub + 1) / p.spc;
   const int64_t v0 = static_cast<int64_t>(rt) * kGRows, d0 = static_cast<int64_t>(dt) * (64 * NBF);
-  const Opnd A = make_opnd(p.P, p.N64, v0, p.Tv, 1, wave, lane);
-  const Opnd B = make_opnd(p.wt, p.N64, d0, p.D, 1, wave, lane);
+  const auto A = [&] {
+    if constexpr (KA) return make_opnd_t<256>(p.ka, v0, wave, lane);
+    else return make_opnd(p.P, p.N64, v0, p.Tv, 1, wave, lane);
+  }();
+  const auto B = [&] {
+    if constexpr (KB) return make_opnd_t<64 * NBF>(p.kb, d0, wave, lane);
+    else return make_opnd(p.wt, p.N64, d0, p.D, 1, wave, lane);
+  }();
   f32x16_t acc[4][NBF];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -912,7 +1076,8 @@ __device__ __attribute__((always_inline)) inline void write_body(const TWritePar
       __syncthreads();
     }
   };
-  gemm_loop(acc, A, B, kb0 * kGK, static_cast<int>(kb1 - kb0), lds, wave, lane, hook);
+  if constexpr (KB) gemm_loop_k(acc, A, B, kb0 * kGK, static_cast<int>(kb1 - kb0), lds, wave, lane);
+  else gemm_loop(acc, A, B, kb0 * kGK, static_cast<int>(kb1 - kb0), lds, wave, lane, hook);
 
   float* dst = p.out_part + static_cast<int64_t>(split) * p.Tv * p.D;
   // (a uniform branch: a select per element kept both forms of every value live)
@@ -955,7 +1120,15 @@ template <int NBF>
 __global__ __launch_bounds__(kGThreads) void tiled_write_batch_kernel(TWriteBatch b) {
   int i = 0;
   for (int k = 1; k < b.n; ++k) i += static_cast<int>(blockIdx.x) >= b.start[k] ? 1 : 0;
-  write_body<NBF, true>(b.p[i], static_cast<int>(blockIdx.x) - b.start[i]);
+  const int bid = static_cast<int>(blockIdx.x) - b.start[i];
+  if (b.p[i].a_rows) write_body<NBF, true, true, true>(b.p[i], bid);
+  else write_body<NBF, true, false, true>(b.p[i], bid);
+}
+// one of the backward's products in a launch of its own
+template <int NBF>
+__global__ __launch_bounds__(kGThreads) void tiled_grad_kernel(TWriteParams p) {
+  if (p.a_rows) write_body<NBF, true, true, true>(p, blockIdx.x);
+  else write_body<NBF, true, false, true>(p, blockIdx.x);
 }
 
 // per-token sums of the gate kernel's partials, in a fixed order:
@@ -1499,8 +1672,11 @@ __global__ __launch_bounds__(kGThreads) void tiled_store_kernel(TStoreParams p) 
 
 // Elementwise passes over 64-row x 64-unit tiles of the [rows, N64] arrays:
 // thread (rp, q) = (tid / 8, tid % 8) owns rows 2 rp, 2 rp + 1 (one token's
-// two routes when paired) and units 8 q .. 8 q + 7; transposed copies go
-// through an LDS tile and leave as 16-byte row pieces.
+// two routes when paired) and units 8 q .. 8 q + 7.  Bound by HBM.  Every
+// array has one layout, rows of units: the gradient products whose k are the
+// rows read it transposed out of LDS (OpndT).  With a second, transposed copy
+// of P, d(xr) and ds the two passes took 285 + 236 us at the Know pool (T =
+// 4 096), without 229 + 204, and the operands' transposes 37.
 constexpr int kTile = 64;
 
 struct ElemTile {
@@ -1530,51 +1706,34 @@ __device__ inline float rowsum8(float v) {
   v += __shfl_xor(v, 4);
   return v;
 }
-// tile[r][c] (bf16 bits, rows = tile rows) -> dst [cols, ld]: column c of the
-// tile is dst row n0 + c, rows r0 .. r0 + nr - 1 (nr a multiple of 8)
-__device__ inline void store_transposed(const uint16_t (*tile)[kTile + 8], int nr, uint16_t* dst, int64_t ld,
-                                        int64_t n0, int64_t r0, int64_t ncols) {
-  for (int idx = threadIdx.x; idx < kTile * (nr / 8); idx += 256) {
-    const int c = idx / (nr / 8), k = idx % (nr / 8);
-    if (n0 + c >= ncols) continue;
-    uint32_t w[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      w[e] = static_cast<uint32_t>(tile[8 * k + 2 * e][c]) | (static_cast<uint32_t>(tile[8 * k + 2 * e + 1][c]) << 16);
-    *reinterpret_cast<u32x4_t*>(dst + (n0 + c) * ld + r0 + 8 * k) = u32x4_t{w[0], w[1], w[2], w[3]};
-  }
-}
-
 struct ElemParams {
   const uint16_t* S;      // [Tv, N64] bf16 scores
   const uint16_t* XR;     // [T, N64] bf16 x.r per token
   const uint16_t* DP;     // [Tv, N64] bf16 dP (E2)
   const float* tau;       // [Tv]
   const float* dden;      // [Tv] (E2)
-  uint16_t* PT;           // [N64, Tv64] P^T (E1)
+  uint16_t* P;            // [Tv, N64] (E1, or E2 with P_OUT)
   float* inten_part;      // [N64 / 64][Tv] sum intensity partials (E1)
   float* psum;            // [Tv64 / 64][N64] column sums of s (E1)
   float* pmax;            // [Tv64 / 64][N64] column maxima of the gate (E1)
   uint16_t* DXR;          // [T, N64] d(xr) per token (E2)
-  uint16_t* DXRT;         // [N64, T64] (E2)
   float* dm_part;         // [N64 / 64][Tv] (E2)
   float* dmz_part;        // [N64 / 64][Tv] sums of dm z (E2, the v4.0.1 gate)
   const float* sdev;      // [Tv] s_std (the v4.0.1 gate's z scale)
-  int64_t Tv, N, N64, Tv64, T64;
+  int64_t Tv, N, N64;
   int routes;
   GateParams gp;
   float exp_scale, sharp;
 };
 
-// E1: the forward's gates from the stored scores and x.r: P^T = bf16(bf16(g) *
-// xr)^T (v41:516-518), per-row sum intensity partials (den, v41:527, 584),
+// E1: the forward's gates from the stored scores and x.r: P = bf16(bf16(g) *
+// xr) (v41:516-518), per-row sum intensity partials (den, v41:527, 584),
 // per-unit column sums of s and maxima of the gate (score_lb / dead penalty,
 // v41:445, 543)
 // GL: the v4.0.1 gate (v401:303-310): the forward kernels' z Phi(z) and, for
 // den = max(sum gate, 1) (v401:340), per-row sums of the gate.
 template <bool GL>
 __global__ __launch_bounds__(256) void bwd_fwd_elem_kernel(ElemParams p) {
-  __shared__ uint16_t tile[kTile][kTile + 8];
   __shared__ float cs[32][kTile + 1], cm[32][kTile + 1];
   const ElemTile et = elem_tile();
   const float c_exp = p.exp_scale, eps = p.gp.eps, maxi = p.gp.maxi;
@@ -1611,12 +1770,7 @@ __global__ __launch_bounds__(256) void bwd_fwd_elem_kernel(ElemParams p) {
       colsum[e] += ok ? s[e] : 0.f;
       colmax[e] = fmaxf(colmax[e], ok ? g : 0.f);
     }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t w = pack_bf16(pr[2 * k], pr[2 * k + 1]);
-      tile[r][8 * et.q + 2 * k] = static_cast<uint16_t>(w);
-      tile[r][8 * et.q + 2 * k + 1] = static_cast<uint16_t>(w >> 16);
-    }
+    if (row_ok) store8_bf16(p.P + v * p.N64 + n, pr);
     isum = rowsum8(isum);
     if (et.q == 0 && row_ok) p.inten_part[static_cast<int64_t>(blockIdx.x) * p.Tv + v] = isum;
   }
@@ -1635,7 +1789,6 @@ __global__ __launch_bounds__(256) void bwd_fwd_elem_kernel(ElemParams p) {
     p.psum[static_cast<int64_t>(blockIdx.y) * p.N64 + et.n0 + threadIdx.x] = a;
     p.pmax[static_cast<int64_t>(blockIdx.y) * p.N64 + et.n0 + threadIdx.x] = m;
   }
-  store_transposed(tile, kTile, p.PT, p.Tv64, et.n0, et.v0, p.N64);
 }
 
 // The gate derivative of one element (v41:506-518) from its bf16 score s,
@@ -1702,15 +1855,12 @@ __device__ inline GateGradGl gate_grad_gl(float s, float x, float dp, float tau,
 
 // E2: the gate derivative from the stored scores, x.r and dP: per-row sums of
 // dm (the tau chain's input) and d(xr), summed over the routes of a token
-// (the broadcast of x.r, v41:796-797) and stored in both layouts.  dm itself
-// is not stored: the ds pass recomputes it from the same bf16 inputs (reading
+// (the broadcast of x.r, v41:796-797).  dm itself is not stored: the ds pass recomputes it from the same bf16 inputs (reading
 // three bf16 arrays costs less than writing and reading an fp32 one).
-// PT_OUT (the forward's den and unit statistics given, no E1 pass): also P^T
-// = bf16(gate_bf * xr)^T (v41:516-518) from the same gate.
-template <bool PT_OUT, bool GL = false>
+// P_OUT (the forward's den and unit statistics given, no E1 pass): also P =
+// bf16(gate_bf * xr) (v41:516-518) from the same gate.
+template <bool P_OUT, bool GL = false>
 __global__ __launch_bounds__(256) void bwd_gate_elem_kernel(ElemParams p) {
-  __shared__ uint16_t tile[kTile][kTile + 8];
-  __shared__ uint16_t ptile[PT_OUT ? kTile : 1][kTile + 8];
   const ElemTile et = elem_tile();
   const int64_t n = et.n0 + 8 * et.q;
   float dxs[2][8];
@@ -1747,14 +1897,8 @@ __global__ __launch_bounds__(256) void bwd_gate_elem_kernel(ElemParams p) {
       sdm += ok ? dm : 0.f;
       pr[e] = ok ? gb * x[e] : 0.f;  // bf16 product, rounded by the packing below
     }
-    if constexpr (PT_OUT) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t w = pack_bf16(pr[2 * k], pr[2 * k + 1]);
-        ptile[r][8 * et.q + 2 * k] = static_cast<uint16_t>(w);
-        ptile[r][8 * et.q + 2 * k + 1] = static_cast<uint16_t>(w >> 16);
-      }
-    }
+    if constexpr (P_OUT)
+      if (row_ok) store8_bf16(p.P + v * p.N64 + n, pr);
     sdm = rowsum8(sdm);
     if (et.q == 0 && row_ok) p.dm_part[static_cast<int64_t>(blockIdx.x) * p.Tv + v] = sdm;
     if constexpr (GL) {
@@ -1763,7 +1907,6 @@ __global__ __launch_bounds__(256) void bwd_gate_elem_kernel(ElemParams p) {
     }
   }
   // d(xr) per token: one row per route (single) or the pair's sum (paired)
-  const int nt = p.routes == 2 ? kTile / 2 : kTile;  // tokens in this tile
   const int64_t t0 = p.routes == 2 ? et.v0 / 2 : et.v0;
   const int64_t T = p.Tv / p.routes;
 #pragma unroll
@@ -1773,17 +1916,8 @@ __global__ __launch_bounds__(256) void bwd_gate_elem_kernel(ElemParams p) {
     float o[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = p.routes == 2 ? dxs[0][e] + dxs[1][e] : dxs[rr][e];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t w = pack_bf16(o[2 * k], o[2 * k + 1]);
-      tile[tr][8 * et.q + 2 * k] = static_cast<uint16_t>(w);
-      tile[tr][8 * et.q + 2 * k + 1] = static_cast<uint16_t>(w >> 16);
-    }
     if (t0 + tr < T) store8_bf16(p.DXR + (t0 + tr) * p.N64 + n, o);
   }
-  __syncthreads();
-  store_transposed(tile, nt, p.DXRT, p.T64, et.n0, t0, p.N64);
-  if constexpr (PT_OUT) store_transposed(ptile, kTile, p.PT, p.Tv64, et.n0, et.v0, p.N64);
 }
 
 struct DsParams {
@@ -1798,10 +1932,9 @@ struct DsParams {
   const float* dead;    // [N64]
   const float* coef;    // {c0, c1}
   uint16_t* DS;         // [Tv, N64]
-  uint16_t* DST;        // [N64, Tv64]
   const float* sdev;    // [Tv] s_std (the v4.0.1 gate)
   float d_pen;
-  int64_t Tv, N, N64, Tv64;
+  int64_t Tv, N, N64;
   int routes;
   GateParams gp;
   float exp_scale, sharp;
@@ -1809,11 +1942,10 @@ struct DsParams {
 
 // E3: ds = bf16(dm + alpha_v + beta_v s + (c0 + c1 pn[n] - d_pen [pn < 0] dead[n]) / Tv)
 // (the tau chain, v41:461-464, and the per-unit score_lb / dead-penalty
-// terms, v41:445-447, 543-552), zero past N; both layouts.  dm as in E2
+// terms, v41:445-447, 543-552), zero past N.  dm as in E2
 // (gate_grad on the same bf16 inputs).
 template <bool GL = false>
 __global__ __launch_bounds__(256) void bwd_ds_elem_kernel(DsParams p) {
-  __shared__ uint16_t tile[kTile][kTile + 8];
   const ElemTile et = elem_tile();
   const int64_t n = et.n0 + 8 * et.q;
   const float c0 = p.coef[0], c1 = p.coef[1];
@@ -1843,16 +1975,8 @@ __global__ __launch_bounds__(256) void bwd_ds_elem_kernel(DsParams p) {
       else dm = gate_grad(s[e], x[e], dp[e], tau, dden, p.gp, p.exp_scale, p.sharp).dm;
       o[e] = row_ok && n + e < p.N ? dm + a + b * s[e] + unit[e] : 0.f;
     }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t w = pack_bf16(o[2 * k], o[2 * k + 1]);
-      tile[r][8 * et.q + 2 * k] = static_cast<uint16_t>(w);
-      tile[r][8 * et.q + 2 * k + 1] = static_cast<uint16_t>(w >> 16);
-    }
     if (row_ok) store8_bf16(p.DS + v * p.N64 + n, o);
   }
-  __syncthreads();
-  store_transposed(tile, kTile, p.DST, p.Tv64, et.n0, et.v0, p.N64);
 }
 
 // sum[v] = sum over b of part[b][v] (fixed order), four partial groups per row
@@ -2066,6 +2190,31 @@ __global__ __launch_bounds__(256) void bwd_sum_kernel(const float* __restrict__ 
   out[i] = round_bf16(a);
 }
 
+// Whole last blocks for the gradient products' k operands (KRows): zero rows
+// [rows, rows64) of the workspace's arrays (src null), and a zero-padded copy
+// of a caller's array's last, partial block.
+struct PadParams {
+  const uint16_t* src[8];
+  uint16_t* dst[8];       // copies: the 64-row block; else the array
+  int64_t rows[8], ld[8];
+  int n;
+};
+__global__ __launch_bounds__(256) void bwd_pad_kernel(PadParams p) {
+  const int i = blockIdx.y;
+  const int64_t rows = p.rows[i], ld = p.ld[i], r0 = rows / kGK * kGK;  // first row of the last block
+  if (rows == r0) return;
+  for (int64_t k = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; k < kGK * ld / 8; k += 256LL * gridDim.x) {
+    const int64_t row = r0 + k / (ld / 8), c = k % (ld / 8) * 8;
+    u32x4_t v = {0u, 0u, 0u, 0u};
+    if (p.src[i]) {
+      if (row < rows) v = *reinterpret_cast<const u32x4_t*>(p.src[i] + row * ld + c);
+      *reinterpret_cast<u32x4_t*>(p.dst[i] + (row - r0) * ld + c) = v;
+    } else if (row >= rows) {
+      *reinterpret_cast<u32x4_t*>(p.dst[i] + row * ld + c) = v;
+    }
+  }
+}
+
 struct BGemm {
   int64_t M, Nc, K;  // out [M, Nc] = A [M, K] . B [Nc, K]^T
   int RT, DT, spc;
@@ -2122,57 +2271,25 @@ void batch_splits(BGemm* const* gs, int n) {
   }
 }
 
-// bf16 src [rows, cols] -> dst [cols, rows_pad] (zero rows past `rows`), 64 x
-// 64 tiles, 16-byte loads along src rows and 16-byte stores along dst rows
-// (cols a multiple of 8)
-__global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* __restrict__ src,
-                                                          uint16_t* __restrict__ dst, int64_t rows,
-                                                          int64_t rows_pad, int64_t cols) {
-  __shared__ uint16_t tile[64][72];
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64, c0 = static_cast<int64_t>(blockIdx.y) * 64;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int idx = threadIdx.x + 256 * k;  // 512 pieces: 64 rows x 8
-    const int r = idx >> 3, q = idx & 7;
-    const int64_t row = r0 + r, col = c0 + 8 * q;
-    u32x4_t v = {0u, 0u, 0u, 0u};
-    if (row < rows && col < cols) v = *reinterpret_cast<const u32x4_t*>(src + row * cols + col);
-    *reinterpret_cast<u32x4_t*>(&tile[r][8 * q]) = v;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int idx = threadIdx.x + 256 * k;  // 512 pieces: 64 dst rows x 8
-    const int c = idx >> 3, q = idx & 7;
-    const int64_t col = c0 + c, row = r0 + 8 * q;
-    if (col >= cols || row >= rows_pad) continue;
-    uint32_t w[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      w[e] = static_cast<uint32_t>(tile[8 * q + 2 * e][c]) | (static_cast<uint32_t>(tile[8 * q + 2 * e + 1][c]) << 16);
-    *reinterpret_cast<u32x4_t*>(dst + col * rows_pad + row) = u32x4_t{w[0], w[1], w[2], w[3]};
-  }
-}
-
-// src [rows, cols] -> dst [cols, rows_pad] (zero rows past `rows`)
-hipError_t transpose(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t rows_pad, int64_t cols,
-                     hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(rows_pad / 64), static_cast<unsigned>((cols + 63) / 64));
-  hipLaunchKernelGGL(transpose16_kernel, grid, dim3(256), 0, s, src, dst, rows, rows_pad, cols);
-  return hipGetLastError();
-}
-
-// out [M, Nc] (fp32, bf16-rounded) = A [M, K] . B [Nc, K]^T, both with row
-// stride ld (elements), zero past K: the write kernel's parameters (one
-// split: the rounded result straight into out; else fp32 partials in part)
-TWriteParams bwd_params(const BGemm& g, const uint16_t* A, const uint16_t* B, int64_t ld, float* part, float* out) {
+// out [M, Nc] (fp32, bf16-rounded) = A . B with B [K, Nc] and A either [M, K]
+// (rows of ld, zero past K) or [K, M] (a null): the write kernel's parameters
+// (one split: the rounded result straight into out; else fp32 partials in
+// part)
+struct BOpnds {
+  const uint16_t* a;
+  int64_t ld;
+  KRows ka, kb;
+};
+TWriteParams bwd_params(const BGemm& g, const BOpnds& o, float* part, float* out) {
   TWriteParams wp{};
-  wp.P = A;
-  wp.wt = B;
+  wp.P = o.a;
+  wp.N64 = o.ld;
+  wp.ka = o.ka;
+  wp.kb = o.kb;
+  wp.a_rows = o.a == nullptr;
   wp.out_part = g.spc == 1 ? out : part;
   wp.Tv = g.M;
   wp.N = g.K;
-  wp.N64 = ld;
   wp.D = g.Nc;
   wp.cs = g.K;
   wp.nc = 1;
@@ -2198,8 +2315,7 @@ hipError_t bwd_sum(const BGemm& g, const float* part, float* out, hipStream_t s)
 // have one width (the products' workgroups then fill the CUs that one
 // product's last round leaves idle), else one launch each; split products'
 // partials (part[i], disjoint) summed after.
-hipError_t bwd_gemms(const BGemm* g, const uint16_t* const* A, const uint16_t* const* B, const int64_t* ld,
-                     float* const* part, float* const* out, int n, hipStream_t s) {
+hipError_t bwd_gemms(const BGemm* g, const BOpnds* o, float* const* part, float* const* out, int n, hipStream_t s) {
   bool same = n <= kWriteBatch;
   for (int i = 1; i < n; ++i) same = same && g[i].nbf == g[0].nbf;
   if (same) {
@@ -2207,7 +2323,7 @@ hipError_t bwd_gemms(const BGemm* g, const uint16_t* const* A, const uint16_t* c
     b.n = n;
     b.start[0] = 0;
     for (int i = 0; i < n; ++i) {
-      b.p[i] = bwd_params(g[i], A[i], B[i], ld[i], part[i], out[i]);
+      b.p[i] = bwd_params(g[i], o[i], part[i], out[i]);
       b.start[i + 1] = b.start[i] + static_cast<int>(bwd_grid(g[i]));
     }
     if (g[0].nbf == 3)
@@ -2220,11 +2336,11 @@ hipError_t bwd_gemms(const BGemm* g, const uint16_t* const* A, const uint16_t* c
     if (e != hipSuccess) return e;
   } else {
     for (int i = 0; i < n; ++i) {
-      const TWriteParams wp = bwd_params(g[i], A[i], B[i], ld[i], part[i], out[i]);
+      const TWriteParams wp = bwd_params(g[i], o[i], part[i], out[i]);
       if (g[i].nbf == 3)
-        hipLaunchKernelGGL((tiled_write_kernel<3, true>), dim3(bwd_grid(g[i])), dim3(kGThreads), gemm_lds(3), s, wp);
+        hipLaunchKernelGGL(tiled_grad_kernel<3>, dim3(bwd_grid(g[i])), dim3(kGThreads), gemm_lds(3), s, wp);
       else
-        hipLaunchKernelGGL((tiled_write_kernel<4, true>), dim3(bwd_grid(g[i])), dim3(kGThreads), kGemmLds, s, wp);
+        hipLaunchKernelGGL(tiled_grad_kernel<4>, dim3(bwd_grid(g[i])), dim3(kGThreads), kGemmLds, s, wp);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
@@ -2237,9 +2353,9 @@ hipError_t bwd_gemms(const BGemm* g, const uint16_t* const* A, const uint16_t* c
 }
 
 struct BLayout {
-  size_t S, XR, DP, DXR, DS, PT, DXRT, DST, ET, RT, HT, XT, DRAWT, DRAW, RN, WN;
+  size_t S, XR, DP, DXR, DS, P, DRAW, RN, WN, xt, ht, rt, et;
   size_t mom, inten_part, dm_part, dmz_part, tokv, psum, pmax, pn, dead, blk, coef, part, total;
-  int64_t Tv, T64, Tv64, N64;
+  int64_t Tv, N64, T64, Tv64;
   int CT, RTv, RTt, NB, TS, nblk;
   int S_st;  // moment partials per row
   BGemm g_dw, g_dh, g_dx, g_de, g_dr;
@@ -2249,14 +2365,14 @@ BLayout blayout(const srw_desc_t& d) {
   BLayout l{};
   const int64_t T = d.T, N = d.n_units, D = d.d_model, dr = d.d_route, R = d.n_routes;
   l.Tv = T * R;
+  l.N64 = (N + kNAlign - 1) / kNAlign * kNAlign;
   l.T64 = (T + kNAlign - 1) / kNAlign * kNAlign;
   l.Tv64 = (l.Tv + kNAlign - 1) / kNAlign * kNAlign;
-  l.N64 = (N + kNAlign - 1) / kNAlign * kNAlign;
   l.CT = static_cast<int>((N + kGRows - 1) / kGRows);
   l.RTv = static_cast<int>((l.Tv + kGRows - 1) / kGRows);
   l.RTt = static_cast<int>((T + kGRows - 1) / kGRows);
   l.NB = static_cast<int>(l.N64 / kTile);   // unit blocks of the elementwise passes
-  l.TS = static_cast<int>(l.Tv64 / kTile);  // row blocks
+  l.TS = static_cast<int>((l.Tv + kTile - 1) / kTile);  // row blocks
   l.nblk = static_cast<int>((l.N64 + 255) / 256);
   l.g_dw = bgemm(N, D, l.Tv);
   l.g_dh = bgemm(l.Tv, dr, N);
@@ -2277,20 +2393,19 @@ BLayout blayout(const srw_desc_t& d) {
     return at;
   };
   const size_t vn = static_cast<size_t>(l.Tv) * l.N64 * 2, tn = static_cast<size_t>(T) * l.N64 * 2;
+  // k operands of the gradient products (P, d(xr), ds, draw): zero rows up to a whole block
+  const size_t vk = static_cast<size_t>(l.Tv64) * l.N64 * 2, tk = static_cast<size_t>(l.T64) * l.N64 * 2;
   l.S = take(vn);
   l.XR = take(tn);
   l.DP = take(vn);
-  l.DXR = take(tn);
-  l.DS = take(vn);
-  l.PT = take(static_cast<size_t>(l.N64) * l.Tv64 * 2);
-  l.DXRT = take(static_cast<size_t>(l.N64) * l.T64 * 2);
-  l.DST = take(static_cast<size_t>(l.N64) * l.Tv64 * 2);
-  l.ET = take(static_cast<size_t>(dr) * l.N64 * 2);
-  l.RT = take(static_cast<size_t>(D) * l.N64 * 2);
-  l.HT = take(static_cast<size_t>(dr) * l.Tv64 * 2);
-  l.XT = take(static_cast<size_t>(D) * l.T64 * 2);
-  l.DRAWT = take(static_cast<size_t>(D) * l.Tv64 * 2);
-  l.DRAW = take(static_cast<size_t>(l.Tv) * D * 2);
+  l.DXR = take(tk);
+  l.DS = take(vk);
+  l.P = take(vk);
+  l.DRAW = take(static_cast<size_t>(l.Tv64) * D * 2);
+  l.xt = take(static_cast<size_t>(kGK) * D * 2);
+  l.ht = take(static_cast<size_t>(kGK) * dr * 2);
+  l.rt = take(static_cast<size_t>(kGK) * D * 2);
+  l.et = take(static_cast<size_t>(kGK) * dr * 2);
   // the v4.0.1 gate: the forward-normalised read and write rows (v401:300-301)
   const bool gl = d.gate == SRW_GATE_GELU_V401;
   l.RN = take(gl ? static_cast<size_t>(N) * D * 2 : 0);
@@ -2357,8 +2472,7 @@ hipError_t tiled_backward(const BackwardArgs& a) {
   auto b16 = [&](size_t off) { return reinterpret_cast<uint16_t*>(a.ws + off); };
   auto f32 = [&](size_t off) { return reinterpret_cast<float*>(a.ws + off); };
   uint16_t *S = b16(l.S), *XR = b16(l.XR), *DP = b16(l.DP), *DXR = b16(l.DXR), *DS = b16(l.DS);
-  uint16_t *PT = b16(l.PT), *DXRT = b16(l.DXRT), *DST = b16(l.DST), *ET = b16(l.ET), *RT = b16(l.RT);
-  uint16_t *HT = b16(l.HT), *XT = b16(l.XT), *DRAWT = b16(l.DRAWT), *DRAW = b16(l.DRAW);
+  uint16_t *P = b16(l.P), *DRAW = b16(l.DRAW);
   float *mom = f32(l.mom), *inten_part = f32(l.inten_part), *dm_part = f32(l.dm_part);
   float *tokv = f32(l.tokv), *psum = f32(l.psum), *pmax = f32(l.pmax), *pn = f32(l.pn), *dead = f32(l.dead);
   float *blk = f32(l.blk), *coef = f32(l.coef), *part = f32(l.part);
@@ -2375,11 +2489,10 @@ hipError_t tiled_backward(const BackwardArgs& a) {
   hipStream_t st = a.stream;
   hipError_t e;
   for (const void* fn : {reinterpret_cast<const void*>(tiled_stats_kernel),
-                         reinterpret_cast<const void*>(tiled_store_kernel),
-                         reinterpret_cast<const void*>(tiled_write_kernel<4>)})
+                         reinterpret_cast<const void*>(tiled_store_kernel)})
     if ((e = set_lds(fn)) != hipSuccess) return e;
-  if ((e = set_lds(reinterpret_cast<const void*>(tiled_write_kernel<3, true>), gemm_lds(3))) != hipSuccess) return e;
-  if ((e = set_lds(reinterpret_cast<const void*>(tiled_write_kernel<4, true>))) != hipSuccess) return e;
+  if ((e = set_lds(reinterpret_cast<const void*>(tiled_grad_kernel<3>), gemm_lds(3))) != hipSuccess) return e;
+  if ((e = set_lds(reinterpret_cast<const void*>(tiled_grad_kernel<4>))) != hipSuccess) return e;
   if ((e = set_lds(reinterpret_cast<const void*>(tiled_write_batch_kernel<3>), gemm_lds(3))) != hipSuccess) return e;
   if ((e = set_lds(reinterpret_cast<const void*>(tiled_write_batch_kernel<4>))) != hipSuccess) return e;
 #define SRW_TRY(expr) \
@@ -2390,12 +2503,6 @@ hipError_t tiled_backward(const BackwardArgs& a) {
     read = b16(l.RN);
     write = b16(l.WN);
   }
-  // operands of the K = units / K = rows contractions, unit- or row-contiguous
-  SRW_TRY(transpose(emb, ET, N, N64, dr, st));
-  SRW_TRY(transpose(read, RT, N, N64, D, st));
-  SRW_TRY(transpose(h, HT, Tv, l.Tv64, dr, st));
-  SRW_TRY(transpose(x, XT, T, l.T64, D, st));
-
   // forward recompute: scores (stored), moments, tau, x.r (stored).  The
   // three [rows, N64] products with K = d_route or d_model (scores, x.r and
   // dP below) run on the moments kernel's tile loop where it takes that K
@@ -2428,33 +2535,30 @@ hipError_t tiled_backward(const BackwardArgs& a) {
     SRW_TRY(store_gemm(read, x, XR, T, T, 1, N, N64, D, st));
   }
 
-  // E1: gates, P^T, sum intensity, per-unit statistics
+  // E1: gates, P, sum intensity, per-unit statistics
   ElemParams ep{};
   ep.S = S;
   ep.XR = XR;
   ep.DP = DP;
   ep.tau = tau;
   ep.dden = dden;
-  ep.PT = PT;
+  ep.P = P;
   ep.inten_part = inten_part;
   ep.psum = psum;
   ep.pmax = pmax;
   ep.DXR = DXR;
-  ep.DXRT = DXRT;
   ep.dm_part = dm_part;
   ep.dmz_part = gl ? f32(l.dmz_part) : nullptr;
   ep.sdev = sdev;
   ep.Tv = Tv;
   ep.N = N;
   ep.N64 = N64;
-  ep.Tv64 = l.Tv64;
-  ep.T64 = l.T64;
   ep.routes = R;
   ep.gp = a.gp;
   ep.exp_scale = exp_scale;
   ep.sharp = d.sharpness;
   const dim3 grid_e(static_cast<unsigned>(l.NB), static_cast<unsigned>(l.TS));
-  // the forward's den and unit statistics given: no E1 pass (P^T comes from
+  // the forward's den and unit statistics given: no E1 pass (P comes from
   // the E2 pass's gates)
   const bool res = a.cot.den && a.cot.unit_diag;
   const float* zs = zsum;
@@ -2506,7 +2610,7 @@ hipError_t tiled_backward(const BackwardArgs& a) {
                      dm_part, ep.dmz_part, l.NB, Tv, N, a.in.tau_offset, mean, var, sdev, a.g.dtau_offset, alpha,
                      beta);
   SRW_TRY(hipGetLastError());
-  // E3: ds in both layouts
+  // E3: ds
   DsParams dp{};
   dp.S = S;
   dp.XR = XR;
@@ -2519,13 +2623,11 @@ hipError_t tiled_backward(const BackwardArgs& a) {
   dp.dead = dead;
   dp.coef = coef;
   dp.DS = DS;
-  dp.DST = DST;
   dp.sdev = sdev;
   dp.d_pen = a.cot.d_dead_penalty;
   dp.Tv = Tv;
   dp.N = N;
   dp.N64 = N64;
-  dp.Tv64 = l.Tv64;
   dp.routes = R;
   dp.gp = a.gp;
   dp.exp_scale = exp_scale;
@@ -2535,12 +2637,37 @@ hipError_t tiled_backward(const BackwardArgs& a) {
   SRW_TRY(hipGetLastError());
 
   // the five gradient contractions: bf16 dots, fp32 accumulation
-  SRW_TRY(transpose(DRAW, DRAWT, Tv, l.Tv64, D, st));
   {
     BGemm gs[5] = {l.g_dw, l.g_dr, l.g_de, l.g_dx, l.g_dh};
-    const uint16_t* As[5] = {PT, DXRT, DST, DXR, DS};
-    const uint16_t* Bs[5] = {DRAWT, XT, HT, RT, ET};
-    int64_t lds_[5] = {l.Tv64, l.T64, l.Tv64, N64, N64};
+    PadParams pp{};
+    auto pad = [&](const uint16_t* src, uint16_t* dst, int64_t rows, int64_t ld) {
+      pp.src[pp.n] = src;
+      pp.dst[pp.n] = dst;
+      pp.rows[pp.n] = rows;
+      pp.ld[pp.n] = ld;
+      if (rows % kGK) ++pp.n;
+    };
+    pad(nullptr, P, Tv, N64);
+    pad(nullptr, DXR, T, N64);
+    pad(nullptr, DS, Tv, N64);
+    pad(nullptr, DRAW, Tv, D);
+    pad(x, b16(l.xt), T, D);
+    pad(h, b16(l.ht), Tv, dr);
+    pad(read, b16(l.rt), N, D);
+    pad(emb, b16(l.et), N, dr);
+    if (pp.n > 0) {
+      hipLaunchKernelGGL(bwd_pad_kernel, dim3(64, static_cast<unsigned>(pp.n)), dim3(256), 0, st, pp);
+      SRW_TRY(hipGetLastError());
+    }
+    auto own = [](const uint16_t* p, int64_t ld) { return KRows{p, ld, nullptr, 0}; };
+    auto user = [](const uint16_t* p, int64_t ld, const uint16_t* tail, int64_t rows) {
+      return KRows{p, ld, rows % kGK ? tail : nullptr, rows / kGK * kGK};
+    };
+    BOpnds os[5] = {{nullptr, 0, own(P, N64), own(DRAW, D)},
+                    {nullptr, 0, own(DXR, N64), user(x, D, b16(l.xt), T)},
+                    {nullptr, 0, own(DS, N64), user(h, dr, b16(l.ht), Tv)},
+                    {DXR, N64, {}, user(read, D, b16(l.rt), N)},
+                    {DS, N64, {}, user(emb, dr, b16(l.et), N)}};
     float* outs[5] = {a.g.dwrite, a.g.dread, a.g.demb, a.g.dx, a.g.dh};
     // the products with the longest workgroups (k blocks per split) first
     // (stable insertion sort of the five)
@@ -2548,18 +2675,16 @@ hipError_t tiled_backward(const BackwardArgs& a) {
     for (int i = 1; i < 5; ++i)
       for (int j = i; j > 0 && wg_blocks(gs[j]) > wg_blocks(gs[j - 1]); --j) {
         std::swap(gs[j], gs[j - 1]);
-        std::swap(As[j], As[j - 1]);
-        std::swap(Bs[j], Bs[j - 1]);
-        std::swap(lds_[j], lds_[j - 1]);
+        std::swap(os[j], os[j - 1]);
         std::swap(outs[j], outs[j - 1]);
       }
     float* parts[5];
-    float* pp = part;
+    float* at = part;
     for (int i = 0; i < 5; ++i) {
-      parts[i] = pp;
-      if (gs[i].spc > 1) pp += al256(static_cast<int64_t>(gs[i].spc) * gs[i].M * gs[i].Nc * 4) / 4;
+      parts[i] = at;
+      if (gs[i].spc > 1) at += al256(static_cast<int64_t>(gs[i].spc) * gs[i].M * gs[i].Nc * 4) / 4;
     }
-    SRW_TRY(bwd_gemms(gs, As, Bs, lds_, parts, outs, 5, st));
+    SRW_TRY(bwd_gemms(gs, os, parts, outs, 5, st));
   }
   if (gl) {  // d read / d write through the forward normalisation
     const dim3 grid_n(static_cast<unsigned>((N + 3) / 4));
