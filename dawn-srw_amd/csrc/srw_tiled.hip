@@ -158,9 +158,19 @@ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) |
 // NBF: B fragments per wave and k-step -- the B tile holds 64 NBF rows (256 or
 // 192), each wave 32 NBF of them, so the output tile is 256 x 64 NBF (192 when
 // the B side is 384 wide: no padded columns).
-template <int NBF, class Hook>
-__device__ inline void gemm_loop(f32x16_t (&acc)[4][NBF], const Opnd& A, const Opnd& B, int64_t k0, int nk,
-                                 char* lds, int wave, int lane, Hook&& hook) {
+// Tail: the last two blocks have a k loop body of their own, in which
+// tail(q, half, stage) takes the place of the loads of blocks nk and nk + 1:
+// load q of 16 into the stage that no wave reads any more (half 0 in block
+// nk's stage, half 1 in block nk + 1's).  The loads of half 1 may still be in
+// flight on return, and both stages are the caller's, without a barrier.
+struct NoTail {
+  __device__ void operator()(int, int, char*) const {}
+};
+template <int NBF, class Hook, class Tail = NoTail>
+__device__ __attribute__((always_inline)) inline void gemm_loop(f32x16_t (&acc)[4][NBF], const Opnd& A, const Opnd& B,
+                                                                int64_t k0, int nk, char* lds, int wave, int lane,
+                                                                Hook&& hook, Tail&& tail = Tail{}) {
+  constexpr bool TAIL = !std::is_same_v<std::remove_reference_t<Tail>, NoTail>;
   constexpr int NB = 64 * NBF;                 // B-tile rows
   constexpr int NL = 8 + NB / 32;              // 16-byte loads per wave and k block
   constexpr int NQ = 4 * NBF;                  // MFMAs per wave and k-step
@@ -188,15 +198,30 @@ __device__ inline void gemm_loop(f32x16_t (&acc)[4][NBF], const Opnd& A, const O
   auto order = [](int r) { return r == 0 ? 0 : (r <= NBF ? 3 + r : r - NBF); };
 #pragma unroll
   for (int q = 0; q < NL; ++q) issue(q, 0, lds);
+  if constexpr (TAIL) {
+    static_assert(NBF == 4, "a tail has 16 loads");
+    if (nk == 1) {
+      wait_vm0();
 #pragma unroll
-  for (int q = 0; q < NL; ++q) issue(q, 1, lds + STAGE);
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(NL));  // block 0 has landed, block 1 is in flight
+      for (int q = 0; q < NL; ++q) tail(q, 0, lds + STAGE);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NL; ++q) issue(q, 1, lds + STAGE);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(NL));
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < NL; ++q) issue(q, 1, lds + STAGE);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(NL));  // block 0 has landed, block 1 is in flight
+  }
   barrier_lds();
   hook(0, lds);
   u32x4_t f[2][NF];
 #pragma unroll
   for (int g = 0; g < NF; ++g) f[0][g] = frag(lds, g, 0);
-  for (int kb = 0; kb < nk; ++kb) {
+  // LEFT: blocks after this one (2: two or more, or no tail)
+  auto block = [&](int kb, auto left_tag) __attribute__((always_inline)) {
+    constexpr int LEFT = decltype(left_tag)::value;
     char* st = lds + (kb & 1) * STAGE;
     char* nxt = lds + ((kb & 1) ^ 1) * STAGE;
 #pragma unroll
@@ -214,21 +239,31 @@ __device__ inline void gemm_loop(f32x16_t (&acc)[4][NBF], const Opnd& A, const O
         // fragment r of the next k-step is read at MFMA r NQ / NF (one per two MFMAs at NBF = 4)
 #pragma unroll
         for (int r = 0; r < NF; ++r) {
-          if (r * NQ / NF == q) {
+          if (r * NQ / NF == q && (m < 3 || LEFT > 0)) {
             const int g = order(r);
             f[cb ^ 1][g] = m < 3 ? frag(st, g, m + 1) : frag(nxt, g, 0);
           }
         }
         if (m == 3) {
 #pragma unroll
-          for (int L = q * NL / NQ; L < (q + 1) * NL / NQ; ++L) issue(L, kb + 2, st);
+          for (int L = q * NL / NQ; L < (q + 1) * NL / NQ; ++L) {
+            if constexpr (LEFT == 2) issue(L, kb + 2, st);
+            else tail(L, 1 - LEFT, st);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  if constexpr (TAIL) {
+    for (int kb = 0; kb < nk - 2; ++kb) block(kb, std::integral_constant<int, 2>{});
+    if (nk > 1) block(nk - 2, std::integral_constant<int, 1>{});
+    block(nk - 1, std::integral_constant<int, 0>{});
+  } else {
+    for (int kb = 0; kb < nk; ++kb) block(kb, std::integral_constant<int, 2>{});
+    wait_vm0();
+    __syncthreads();  // the trailing reloads have landed before LDS is reused
   }
-  wait_vm0();
-  __syncthreads();  // the trailing reloads have landed before LDS is reused
 }
 
 // The same products with the B operand's rows k (OpndT), and A's as they are
@@ -333,6 +368,46 @@ struct NoHook {
   __device__ void operator()(int, char*) const {}
 };
 
+// A wave's 128 rows x 128 units of a [rows, N64] bf16 array, in the stages that
+// the GEMM loop is done with: rows 0-63 in half 0, 64-127 in half 1, 256 bytes
+// a row, the 16-byte piece q of row r in slot q ^ (r & 15).  An accumulator
+// holds four consecutive units per lane, 8 bytes in each of 32 rows: straight
+// to memory, every access touches 32 lines and every line is touched eight
+// times; through here each access is four rows' whole lines, streamed past L2
+// (the array is larger than it).  T = 16 384, N = 100 000, D = dr = 1 024:
+// score kernel 4 002 -> 3 477 us (2 720 without an epilogue), gate kernel,
+// whose scores arrive under the last blocks' products, 5 432 -> 4 787.
+struct RowPatch {
+  char* half[2];
+  int lane;
+  // lane (u, h): units 32 i + 8 q + 4 h .. + 3 of row 32 j + u
+  __device__ uint2* at(int j, int i, int q) const {
+    const int u = lane & 31, h = lane >> 5;
+    return reinterpret_cast<uint2*>(half[j >> 1] + (32 * (j & 1) + u) * 256 + (((4 * i + q) ^ (u & 15)) * 16) + 8 * h);
+  }
+  // piece of load or store n (rows 4 n + lane / 16) that the lane's slot holds
+  __device__ int piece(int n) const { return (lane & 15) ^ (lane >> 4) ^ (4 * (n & 3)); }
+  // rows 32 j .. 32 j + 31 to C (first row t0, first unit c0)
+  __device__ void flush(int j, uint16_t* C, int64_t t0, int64_t rows, int64_t c0, int64_t N64) const {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const u32x4_t w = *reinterpret_cast<const u32x4_t*>(half[j >> 1] + (32 * (j & 1) + 4 * n) * 256 + lane * 16);
+      const int64_t t = t0 + 32 * j + 4 * n + (lane >> 4), c = c0 + 8 * piece(n);
+      if (t < rows && c < N64) __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t*>(C + t * N64 + c));
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+__device__ inline RowPatch row_patch(char* lds, int nk, int wave, int lane) {
+  char* w = lds + wave * (kStageBytes / 4);
+  return RowPatch{{w + (nk & 1) * kStageBytes, w + ((nk & 1) ^ 1) * kStageBytes}, lane};
+}
+// a tail that loads nothing (the epilogue uses the stages)
+struct EndTail {
+  __device__ void operator()(int, int, char*) const {}
+};
+
 // Workgroup -> (row tile, column tile) with the column tile shared by the
 // workgroups of one XCD (blockIdx % 8 on MI355X): they walk the row tiles of
 // one column tile together, so its operand rows are fetched into that XCD's
@@ -394,67 +469,74 @@ __global__ __launch_bounds__(kGThreads) void tiled_stats_kernel(TStatsParams p) 
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x16_t{};
-  gemm_loop(acc, A, B, 0, static_cast<int>(p.dr / kGK), lds, wave, lane, NoHook{});
+  const int nk = static_cast<int>(p.dr / kGK);
+  gemm_loop(acc, A, B, 0, nk, lds, wave, lane, NoHook{}, EndTail{});
+  const RowPatch patch = row_patch(lds, nk, wave, lane);
 
   const int64_t nleft = p.N - (u0 + 128 * wa + 4 * h);  // units of this wave-row left in the pool
+  const bf16x2_t ones = __builtin_bit_cast(bf16x2_t, 0x3f803f80u);
+  // FULL: every unit of the tile is in the pool (all but the last unit tile)
+  auto epilogue = [&](auto full_tag) {
+    constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t t = v0 + 128 * wb + 32 * j + u;
-    uint16_t* srow = p.S + t * p.N64;
-    float s1 = 0.f, s2 = 0.f;
+    for (int j = 0; j < 4; ++j) {
+      const int64_t t = v0 + 128 * wb + 32 * j + u;
+      float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 4; ++i) {
 #pragma unroll
-      for (int v = 0; v < 16; v += 4) {
-        uint32_t sq[2];
+        for (int v = 0; v < 16; v += 4) {
+          uint32_t sq[2];
 #pragma unroll
-        for (int e2 = 0; e2 < 2; ++e2) {
-          const uint32_t sp = pack_bf16(acc[i][j][v + 2 * e2], acc[i][j][v + 2 * e2 + 1]);  // bf16 scores (v41:439)
-          float a = lo_f32(sp), b = hi_f32(sp);
-          const int r = 32 * i + 8 * (v >> 2) + 2 * e2;  // unit offset from u0 + 128 wa + 4 h
-          const bool oka = r < nleft, okb = r + 1 < nleft;
-          a = oka ? a : 0.f;
-          b = okb ? b : 0.f;
-          s1 += a;
-          s2 += __fmul_rn(a, a);
-          s1 += b;
-          s2 += __fmul_rn(b, b);
-          sq[e2] = pack_bf16(a, b);
+          for (int e2 = 0; e2 < 2; ++e2) {
+            uint32_t sp = pack_bf16(acc[i][j][v + 2 * e2], acc[i][j][v + 2 * e2 + 1]);  // bf16 scores (v41:439)
+            if constexpr (!FULL) {
+              const int r = 32 * i + 8 * (v >> 2) + 2 * e2;  // unit offset from u0 + 128 wa + 4 h
+              sp = r + 1 < nleft ? sp : (r < nleft ? sp & 0xffffu : 0u);
+            }
+            // sum s and sum s^2 of the pair, one v_dot2_f32_bf16 each
+            const bf16x2_t sb = __builtin_bit_cast(bf16x2_t, sp);
+            s1 = __builtin_amdgcn_fdot2_f32_bf16(sb, ones, s1, false);
+            if (!p.centred) s2 = __builtin_amdgcn_fdot2_f32_bf16(sb, sb, s2, false);
+            sq[e2] = sp;
+          }
+          *patch.at(j, i, v >> 2) = make_uint2(sq[0], sq[1]);
         }
-        const int64_t n0 = u0 + 128 * wa + 32 * i + 8 * (v >> 2) + 4 * h;
-        if (t < p.Tv && n0 < p.N64) {
-          typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-          *reinterpret_cast<u32x2_t*>(srow + n0) = u32x2_t{sq[0], sq[1]};
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    s1 += __shfl_xor(s1, 32);
-    if (p.centred) {
-      // sum (s - mean)^2 over these units' bf16 scores, their mean from s1
-      // (v41:1719-1721 over a 128-unit slice; merged in srw_tau_kernel)
-      const int64_t nrow = p.N - (u0 + 128 * wa);
-      const float n = static_cast<float>(nrow <= 0 ? 0 : (nrow < 128 ? nrow : 128));
-      const float mu = n > 0.f ? s1 / n : 0.f;
-      s2 = 0.f;
+      patch.flush(j, p.S, v0 + 128 * wb, p.Tv, u0 + 128 * wa, p.N64);
+      s1 += __shfl_xor(s1, 32);
+      if (p.centred) {
+        // sum (s - mean)^2 over these units' bf16 scores, their mean from s1
+        // (v41:1719-1721 over a 128-unit slice; merged in srw_tau_kernel)
+        const int64_t nrow = p.N - (u0 + 128 * wa);
+        const float n = static_cast<float>(nrow <= 0 ? 0 : (nrow < 128 ? nrow : 128));
+        const float mu = n > 0.f ? s1 / n : 0.f;
+        s2 = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; v += 2) {
-          const uint32_t sp = pack_bf16(acc[i][j][v], acc[i][j][v + 1]);
-          const int r = 32 * i + 8 * (v >> 2) + (v & 3);
-          const float da = r < nleft ? lo_f32(sp) - mu : 0.f, db = r + 1 < nleft ? hi_f32(sp) - mu : 0.f;
-          s2 += __fmul_rn(da, da);
-          s2 += __fmul_rn(db, db);
-        }
+          for (int v = 0; v < 16; v += 2) {
+            const uint32_t sp = pack_bf16(acc[i][j][v], acc[i][j][v + 1]);
+            const int r = 32 * i + 8 * (v >> 2) + (v & 3);
+            const float da = FULL || r < nleft ? lo_f32(sp) - mu : 0.f;
+            const float db = FULL || r + 1 < nleft ? hi_f32(sp) - mu : 0.f;
+            s2 += __fmul_rn(da, da);
+            s2 += __fmul_rn(db, db);
+          }
+      }
+      s2 += __shfl_xor(s2, 32);
+      if (h == 0 && t < p.Tv) {
+        float* m = p.mom + ((static_cast<int64_t>(2 * ct + wa)) * p.Tv + t) * 2;
+        m[0] = s1;
+        m[1] = s2;
+      }
     }
-    s2 += __shfl_xor(s2, 32);
-    if (h == 0 && t < p.Tv) {
-      float* m = p.mom + ((static_cast<int64_t>(2 * ct + wa)) * p.Tv + t) * 2;
-      m[0] = s1;
-      m[1] = s2;
-    }
-  }
+  };
+  if (u0 + kGRows <= p.N)
+    epilogue(std::true_type{});
+  else
+    epilogue(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -465,8 +547,6 @@ struct TGateParams {
   const uint16_t* read;  // [N, D]
   const float* tau;      // [Tv]
   uint16_t* P;           // [Tv, N64]: the bf16 scores in, P out (in place)
-  uint16_t* P_out;       // KEEP: P here instead, the scores stay in P
-  uint16_t* XR_out;      // KEEP: bf16 x.r [Tv, N64]
   float* tok_part;       // [2 CT][Tv][4]: sum gate, sum intensity, active count
   uint32_t* mask32;      // [Tv][mask_words32] or null
   float* G;              // [Tv, N] every unit's fp32 gate (SRW_FLAG_GATE_OUT) or null
@@ -477,11 +557,10 @@ struct TGateParams {
   float exp_scale;       // -sharpness * log2(e)
 };
 
-// KEEP (the backward's recompute): P and x.r go to P_out / XR_out and the
-// stored scores stay.  GOUT: every unit's fp32 gate also goes to G (a
-// variant of its own: the per-element stores and their addresses would
-// otherwise sit in every call's epilogue code).
-template <bool KEEP, bool GOUT = false>
+// GOUT: every unit's fp32 gate also goes to G (a variant of its own: the
+// per-element stores and their addresses would otherwise sit in every call's
+// epilogue code).
+template <bool GOUT>
 __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -495,11 +574,22 @@ __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x16_t{};
+  const int nk = static_cast<int>(p.D / kGK);
+  const RowPatch patch = row_patch(lds, nk, wave, lane);
   {
     const Opnd A = make_opnd(p.read, p.D, u0, p.N, 1, wave, lane);
     const Opnd B = make_opnd(p.x, p.D, v0, p.Tv, p.routes, wave, lane);
-    gemm_loop(acc, A, B, 0, static_cast<int>(p.D / kGK), lds, wave, lane, NoHook{});
+    // the scores, under the last blocks' products (rows and columns past the end: some in bounds)
+    const char* sbase = reinterpret_cast<const char*>(p.P + v0 * p.N64);
+    auto scores = [&](int q, int half, char* stage) __attribute__((always_inline)) {
+      const int64_t row = v0 + 128 * wb + 64 * half + 4 * q + (lane >> 4), col = u0 + 128 * wa + 8 * patch.piece(q);
+      const uint32_t off = static_cast<uint32_t>((row < p.Tv ? row : p.Tv - 1) - v0) * static_cast<uint32_t>(2 * p.N64) +
+                           static_cast<uint32_t>(2 * (col < p.N64 ? col : p.N64 - 8));
+      g2lds16(sbase + off, stage + wave * (kStageBytes / 4) + q * 1024);
+    };
+    gemm_loop(acc, A, B, 0, nk, lds, wave, lane, NoHook{}, scores);
   }
+  wait_vm0();
 
   // gate epilogue (v41:503-534): margin = s - tau - thr folded into
   // arg = s * c + k (c = -sharpness log2 e), sigmoid = 1 / (1 + 2^arg),
@@ -515,7 +605,6 @@ __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
     for (int j = 0; j < 4; ++j) {
       const int64_t t = v0 + 128 * wb + 32 * j + u;
       const bool tok = t < p.Tv;
-      uint16_t* prow = p.P + (tok ? t : p.Tv - 1) * p.N64;
       const float tau_thr = p.tau[tok ? t : p.Tv - 1] + p.gp.thr;
       const float k_exp = -tau_thr * c_exp;
       const float tau_cut = tau_thr + p.gp.cut;
@@ -524,10 +613,12 @@ __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int64_t nb = u0 + 128 * wa + 32 * i + 4 * h;
-        u32x2_t sv[4], xv[4];
+        u32x2_t sv[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)  // the last unit tile may reach past the row's N64 columns
-          sv[q] = FULL || nb + 8 * q < p.N64 ? *reinterpret_cast<const u32x2_t*>(prow + nb + 8 * q) : u32x2_t{0u, 0u};
+        for (int q = 0; q < 4; ++q) {
+          const uint2 w = *patch.at(j, i, q);
+          sv[q] = u32x2_t{w.x, w.y};
+        }
         uint32_t bits = 0;  // element v of the 16 at bit 15 - v: set <=> arg < 0 <=> act > 0.5
 #pragma unroll
         for (int v = 0; v < 16; v += 2) {
@@ -555,21 +646,10 @@ __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
           }
           const uint32_t gq = pack_bf16(g2[0], g2[1]);                              // gate_bf (v41:516)
           const uint32_t xq = pack_bf16(acc[i][j][v], acc[i][j][v + 1]);            // xr (v41:517)
-          if constexpr (KEEP) xv[v >> 2][(v >> 1) & 1] = xq;
           sv[v >> 2][(v >> 1) & 1] = pack_bf16(lo_f32(gq) * lo_f32(xq), hi_f32(gq) * hi_f32(xq));  // (v41:518)
         }
-        if (tok) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            if (!(FULL || nb + 8 * q < p.N64)) continue;
-            if constexpr (KEEP) {
-              *reinterpret_cast<u32x2_t*>(p.P_out + t * p.N64 + nb + 8 * q) = sv[q];
-              *reinterpret_cast<u32x2_t*>(p.XR_out + t * p.N64 + nb + 8 * q) = xv[q];
-            } else {
-              *reinterpret_cast<u32x2_t*>(prow + nb + 8 * q) = sv[q];
-            }
-          }
-        }
+        for (int q = 0; q < 4; ++q) *patch.at(j, i, q) = make_uint2(sv[q][0], sv[q][1]);
         // element v -> unit 8 (v / 4) + 4 h + v % 4 of the 32-unit block
         const uint32_t b = __builtin_bitreverse32(bits) >> 16;  // element v at bit v
         uint32_t m = (b & 0xFu) | ((b & 0xF0u) << 4) | ((b & 0xF00u) << 8) | ((b & 0xF000u) << 12);
@@ -580,6 +660,7 @@ __global__ __launch_bounds__(kGThreads) void tiled_gate_kernel(TGateParams p) {
         if (p.mask32 && h == 0 && tok && word < p.mask_words32) p.mask32[t * p.mask_words32 + word] = m;
         __builtin_amdgcn_sched_barrier(0);  // one accumulator at a time: keeps the live registers bounded
       }
+      patch.flush(j, p.P, v0 + 128 * wb, p.Tv, u0 + 128 * wa, p.N64);
       gs += __shfl_xor(gs, 32);
       is += __shfl_xor(is, 32);
       na += __shfl_xor(na, 32);
@@ -1413,7 +1494,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   static_assert(kGemmLds <= 160 * 1024, "LDS per workgroup");
   for (const void* fn : {reinterpret_cast<const void*>(tiled_stats_kernel),
                          reinterpret_cast<const void*>(tiled_gate_kernel<false>),
-                         reinterpret_cast<const void*>(tiled_gate_kernel<false, true>),
+                         reinterpret_cast<const void*>(tiled_gate_kernel<true>),
                          reinterpret_cast<const void*>(tiled_write_kernel<4>)})
     if ((e = set_lds(fn)) != hipSuccess) return e;
 
@@ -1490,7 +1571,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   gp.exp_scale = exp_scale;
   dominant_kernel_begin(a.stream);
   if (gp.G)
-    hipLaunchKernelGGL((tiled_gate_kernel<false, true>), dim3(grid_rc), dim3(kGThreads), kGemmLds, a.stream, gp);
+    hipLaunchKernelGGL((tiled_gate_kernel<true>), dim3(grid_rc), dim3(kGThreads), kGemmLds, a.stream, gp);
   else
     hipLaunchKernelGGL(tiled_gate_kernel<false>, dim3(grid_rc), dim3(kGThreads), kGemmLds, a.stream, gp);
   dominant_kernel_end(a.stream);
@@ -1638,7 +1719,7 @@ __global__ __launch_bounds__(kGThreads) void tiled_store_kernel(TStoreParams p) 
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wa = wave >> 1, wb = wave & 1, u = lane & 31, h = lane >> 5;
+  const int wa = wave >> 1, wb = wave & 1, nk = static_cast<int>(p.K / kGK);
   int rt, ct;
   if (!tile_of(p.RT, p.CT, rt, ct)) return;
   const int64_t u0 = static_cast<int64_t>(ct) * kGRows, v0 = static_cast<int64_t>(rt) * kGRows;
@@ -1650,23 +1731,18 @@ __global__ __launch_bounds__(kGThreads) void tiled_store_kernel(TStoreParams p) 
   {
     const Opnd A = make_opnd(p.A, p.K, u0, p.N, 1, wave, lane);
     const Opnd B = make_opnd(p.B, p.K, v0, p.rows, p.div, wave, lane);
-    gemm_loop(acc, A, B, 0, static_cast<int>(p.K / kGK), lds, wave, lane, NoHook{});
+    gemm_loop(acc, A, B, 0, nk, lds, wave, lane, NoHook{}, EndTail{});
   }
-  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+  const RowPatch patch = row_patch(lds, nk, wave, lane);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int64_t t = v0 + 128 * wb + 32 * j + u;
-    if (t >= p.rows) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int v = 0; v < 16; v += 4) {
-        const int64_t n0 = u0 + 128 * wa + 32 * i + 8 * (v >> 2) + 4 * h;
-        if (n0 < p.N64)
-          *reinterpret_cast<u32x2_t*>(p.C + t * p.N64 + n0) =
-              u32x2_t{pack_bf16(acc[i][j][v], acc[i][j][v + 1]), pack_bf16(acc[i][j][v + 2], acc[i][j][v + 3])};
-      }
-    }
+      for (int v = 0; v < 16; v += 4)
+        *patch.at(j, i, v >> 2) = make_uint2(pack_bf16(acc[i][j][v], acc[i][j][v + 1]),
+                                             pack_bf16(acc[i][j][v + 2], acc[i][j][v + 3]));
+    patch.flush(j, p.C, v0 + 128 * wb, p.rows, u0 + 128 * wa, p.N64);
   }
 }
 
