@@ -21,11 +21,18 @@ __host__ __device__ inline float bf16_to_f32(uint16_t b) {
   return __builtin_bit_cast(float, static_cast<uint32_t>(b) << 16);
 }
 
+// Round to nearest even.  On the device v_cvt_pk_bf16_f32: the integer form
+// compiles to a branch per value (its NaN case) and bound the backward's
+// elementwise passes.
 __host__ __device__ inline uint16_t f32_to_bf16_bits(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+#else
   uint32_t u = __builtin_bit_cast(uint32_t, f);
   if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);  // quiet NaN
   u += 0x7fffu + ((u >> 16) & 1u);
   return static_cast<uint16_t>(u >> 16);
+#endif
 }
 
 __host__ __device__ inline float round_bf16(float f) { return bf16_to_f32(f32_to_bf16_bits(f)); }

@@ -2055,6 +2055,165 @@ __global__ __launch_bounds__(256) void bwd_ds_elem_kernel(DsParams p) {
   }
 }
 
+// unit[n] = (c0 + c1 pn[n] - d_pen [pn < 0] dead[n]) / Tv over pn in place: E3's
+// per-unit term, for bwd_row_kernel
+__global__ __launch_bounds__(256) void bwd_unit_term_kernel(float* __restrict__ pn, const float* __restrict__ dead,
+                                                            const float* __restrict__ coef, float d_pen, int64_t Tv,
+                                                            int64_t N64) {
+  const int64_t n = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (n >= N64) return;
+  const float pv = pn[n];
+  pn[n] = (coef[0] + coef[1] * pv + (pv < 0.f ? -d_pen * dead[n] : 0.f)) * (1.0f / static_cast<float>(Tv));
+}
+
+// E2, the tau chain and E3 in one: a workgroup owns one token's rows (RT
+// routes), holds their scores and dm in registers (thread i: chunks i, i + TH,
+// ... of eight units, C of them) and so reads S, x.r and dP once; two passes
+// read them twice, because ds needs the row's sum of dm.  Bound by HBM.
+// Know pool, T = 4 096: the training step 1 694 -> 1 472 us (v4.0.1 2 140 -> 1 958),
+// with the roundings in hardware; the passes and bwd_token_kernel took 229 + 204 + 15 before.
+struct RowParams {
+  ElemParams e;         // S, XR, DP, tau, dden, P (or null), DXR, sdev, sizes, gate
+  const float* tau_off;
+  const float* mean;    // [Tv]
+  const float* var;     // [Tv]
+  const float* unit;    // [N64]
+  float* dtau_off;      // [Tv]
+  uint16_t* DS;         // [Tv, N64]
+};
+template <int C, int TH, int RT, bool GL>
+__global__ __launch_bounds__(TH, TH == 256 ? 4 : TH / 128) void bwd_row_kernel(RowParams q) {
+  const ElemParams& p = q.e;
+  constexpr int W = TH / 64, NS = GL ? 2 : 1;
+  __shared__ float red[RT * NS][W];
+  const int tid = threadIdx.x, nch = static_cast<int>(p.N64 >> 3);
+  const int64_t t = blockIdx.x;
+  u32x4_t s[RT][C], x[C], d[RT][C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int64_t n = 8 * static_cast<int64_t>(min(tid + i * TH, nch - 1));  // in bounds; unused past the last chunk
+    x[i] = *reinterpret_cast<const u32x4_t*>(p.XR + t * p.N64 + n);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      s[r][i] = *reinterpret_cast<const u32x4_t*>(p.S + (RT * t + r) * p.N64 + n);
+      d[r][i] = *reinterpret_cast<const u32x4_t*>(p.DP + (RT * t + r) * p.N64 + n);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float dm[RT][C][8], sdm[RT], sdmz[RT], tau[RT], dden[RT], istd[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    sdm[r] = sdmz[r] = 0.f;
+    tau[r] = p.tau[RT * t + r];
+    dden[r] = p.dden[RT * t + r];
+    istd[r] = GL ? 1.0f / p.sdev[RT * t + r] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = tid + i * TH;
+    const int n = 8 * c;
+    float dxs[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dxs[e] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      float pr[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bool ok = n + e < p.N;
+        const float sv = e & 1 ? hi_f32(s[r][i][e / 2]) : lo_f32(s[r][i][e / 2]);
+        const float xv = e & 1 ? hi_f32(x[i][e / 2]) : lo_f32(x[i][e / 2]);
+        const float dv = e & 1 ? hi_f32(d[r][i][e / 2]) : lo_f32(d[r][i][e / 2]);
+        float dx, gb;
+        if constexpr (GL) {
+          const GateGradGl gg = gate_grad_gl(sv, xv, dv, tau[r], istd[r], dden[r]);
+          dm[r][i][e] = gg.dm;
+          dx = gg.dx;
+          gb = gg.gb;
+          sdmz[r] += ok ? gg.dmz : 0.f;
+        } else {
+          const GateGrad gg = gate_grad(sv, xv, dv, tau[r], dden[r], p.gp, p.exp_scale, p.sharp);
+          dm[r][i][e] = gg.dm;
+          dx = gg.dx;
+          gb = gg.gb;
+        }
+        sdm[r] += ok ? dm[r][i][e] : 0.f;
+        asm volatile("" : "+v"(dm[r][i][e]), "+v"(sdm[r]), "+v"(sdmz[r]));  // formed here, not where ds uses it
+        dxs[e] += ok ? dx : 0.f;
+        pr[e] = ok ? gb * xv : 0.f;  // bf16 product, rounded by the packing
+      }
+      if (p.P && c < nch) store8_bf16(p.P + (RT * t + r) * p.N64 + n, pr);
+      __builtin_amdgcn_sched_barrier(0);  // one chunk at a time: interleaved ones spill
+    }
+    if (c < nch) store8_bf16(p.DXR + t * p.N64 + n, dxs);
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const float a = wave_sum(sdm[r]);
+    if ((tid & 63) == 0) red[r * NS][tid >> 6] = a;
+    if constexpr (GL) {
+      const float z = wave_sum(sdmz[r]);
+      if ((tid & 63) == 0) red[r * NS + 1][tid >> 6] = z;
+    }
+  }
+  __syncthreads();
+  float alpha[RT], beta[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {  // the tau chain, as in bwd_token_kernel
+    const int64_t v = RT * t + r;
+    float sa = 0.f, sz = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      sa += red[r * NS][w];
+      if constexpr (GL) sz += red[r * NS + 1][w];
+    }
+    const float fN = static_cast<float>(p.N), mean = q.mean[v];
+    const float dtau = -sa;
+    if (tid == 0) q.dtau_off[v] = dtau * p.sdev[v];
+    const float dstd = dtau * q.tau_off[v] - sz;
+    const float dvar = dstd / (2.0f * sqrtf(q.var[v]));
+    const float dmean = dtau - 2.0f * mean * dvar;
+    alpha[r] = dmean / fN;
+    beta[r] = 2.0f * dvar / fN;
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = tid + i * TH;
+    const int64_t n = 8 * static_cast<int64_t>(c);
+    if (c >= nch) break;
+    const float4 u0 = *reinterpret_cast<const float4*>(q.unit + n), u1 = *reinterpret_cast<const float4*>(q.unit + n + 4);
+    const float unit[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      asm volatile("" : "+v"(s[r][i]));  // unpacked again: kept unpacked, a chunk's scores take eight registers, not four
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float sv = e & 1 ? hi_f32(s[r][i][e / 2]) : lo_f32(s[r][i][e / 2]);
+        o[e] = n + e < p.N ? dm[r][i][e] + alpha[r] + beta[r] * sv + unit[e] : 0.f;
+      }
+      store8_bf16(q.DS + (RT * t + r) * p.N64 + n, o);
+    }
+  }
+}
+
+// Units up to which a row fits the registers of 512 threads (twelve a chunk and
+// route, 128 a thread without spilling, two workgroups a CU); longer rows: two passes.
+constexpr int64_t row_max_units(int routes) { return 8 * 512 * (routes == 2 ? 3 : 7); }
+template <int RT, bool GL>
+void launch_rows(const RowParams& q, hipStream_t st) {
+  const int64_t nch = q.e.N64 / 8;
+  const dim3 grid(static_cast<unsigned>(q.e.Tv / RT));
+  if (nch <= 256) hipLaunchKernelGGL((bwd_row_kernel<1, 256, RT, GL>), grid, dim3(256), 0, st, q);
+  else if (nch <= 512) hipLaunchKernelGGL((bwd_row_kernel<1, 512, RT, GL>), grid, dim3(512), 0, st, q);
+  else if (nch <= 1024) hipLaunchKernelGGL((bwd_row_kernel<2, 512, RT, GL>), grid, dim3(512), 0, st, q);
+  else if (nch <= 1536) hipLaunchKernelGGL((bwd_row_kernel<3, 512, RT, GL>), grid, dim3(512), 0, st, q);
+  else if constexpr (RT == 1) {
+    if (nch <= 2560) hipLaunchKernelGGL((bwd_row_kernel<5, 512, RT, GL>), grid, dim3(512), 0, st, q);
+    else hipLaunchKernelGGL((bwd_row_kernel<7, 512, RT, GL>), grid, dim3(512), 0, st, q);
+  }
+}
+
 // sum[v] = sum over b of part[b][v] (fixed order), four partial groups per row
 __global__ __launch_bounds__(256) void bwd_rowsum_kernel(const float* __restrict__ part, int nb, int64_t rows,
                                                          float* __restrict__ sum) {
@@ -2673,44 +2832,56 @@ hipError_t tiled_backward(const BackwardArgs& a) {
     SRW_TRY(store_gemm(write, DRAW, DP, Tv, Tv, 1, N, N64, D, st));
   }
   dominant_kernel_end(st);
-  if (res && gl)
-    hipLaunchKernelGGL((bwd_gate_elem_kernel<true, true>), grid_e, dim3(256), 0, st, ep);
-  else if (res)
-    hipLaunchKernelGGL(bwd_gate_elem_kernel<true>, grid_e, dim3(256), 0, st, ep);
-  else if (gl)
-    hipLaunchKernelGGL((bwd_gate_elem_kernel<false, true>), grid_e, dim3(256), 0, st, ep);
-  else
-    hipLaunchKernelGGL(bwd_gate_elem_kernel<false>, grid_e, dim3(256), 0, st, ep);
-  SRW_TRY(hipGetLastError());
-  hipLaunchKernelGGL(bwd_token_kernel, dim3(static_cast<unsigned>((Tv + kTokRows - 1) / kTokRows)), dim3(256), 0, st,
-                     dm_part, ep.dmz_part, l.NB, Tv, N, a.in.tau_offset, mean, var, sdev, a.g.dtau_offset, alpha,
-                     beta);
-  SRW_TRY(hipGetLastError());
-  // E3: ds
-  DsParams dp{};
-  dp.S = S;
-  dp.XR = XR;
-  dp.DP = DP;
-  dp.tau = tau;
-  dp.dden = dden;
-  dp.alpha = alpha;
-  dp.beta = beta;
-  dp.pn = pn;
-  dp.dead = dead;
-  dp.coef = coef;
-  dp.DS = DS;
-  dp.sdev = sdev;
-  dp.d_pen = a.cot.d_dead_penalty;
-  dp.Tv = Tv;
-  dp.N = N;
-  dp.N64 = N64;
-  dp.routes = R;
-  dp.gp = a.gp;
-  dp.exp_scale = exp_scale;
-  dp.sharp = d.sharpness;
-  if (gl) hipLaunchKernelGGL(bwd_ds_elem_kernel<true>, grid_e, dim3(256), 0, st, dp);
-  else hipLaunchKernelGGL(bwd_ds_elem_kernel<false>, grid_e, dim3(256), 0, st, dp);
-  SRW_TRY(hipGetLastError());
+  if (N64 <= row_max_units(R)) {
+    float* unit = pn;
+    hipLaunchKernelGGL(bwd_unit_term_kernel, dim3(static_cast<unsigned>((N64 + 255) / 256)), dim3(256), 0, st, unit,
+                       dead, coef, a.cot.d_dead_penalty, Tv, N64);
+    SRW_TRY(hipGetLastError());
+    RowParams q{ep, a.in.tau_offset, mean, var, unit, a.g.dtau_offset, DS};
+    if (!res) q.e.P = nullptr;  // E1 wrote it
+    if (R == 2) gl ? launch_rows<2, true>(q, st) : launch_rows<2, false>(q, st);
+    else gl ? launch_rows<1, true>(q, st) : launch_rows<1, false>(q, st);
+    SRW_TRY(hipGetLastError());
+  } else {
+    if (res && gl)
+      hipLaunchKernelGGL((bwd_gate_elem_kernel<true, true>), grid_e, dim3(256), 0, st, ep);
+    else if (res)
+      hipLaunchKernelGGL(bwd_gate_elem_kernel<true>, grid_e, dim3(256), 0, st, ep);
+    else if (gl)
+      hipLaunchKernelGGL((bwd_gate_elem_kernel<false, true>), grid_e, dim3(256), 0, st, ep);
+    else
+      hipLaunchKernelGGL(bwd_gate_elem_kernel<false>, grid_e, dim3(256), 0, st, ep);
+    SRW_TRY(hipGetLastError());
+    hipLaunchKernelGGL(bwd_token_kernel, dim3(static_cast<unsigned>((Tv + kTokRows - 1) / kTokRows)), dim3(256), 0, st,
+                       dm_part, ep.dmz_part, l.NB, Tv, N, a.in.tau_offset, mean, var, sdev, a.g.dtau_offset, alpha,
+                       beta);
+    SRW_TRY(hipGetLastError());
+    // E3: ds
+    DsParams dp{};
+    dp.S = S;
+    dp.XR = XR;
+    dp.DP = DP;
+    dp.tau = tau;
+    dp.dden = dden;
+    dp.alpha = alpha;
+    dp.beta = beta;
+    dp.pn = pn;
+    dp.dead = dead;
+    dp.coef = coef;
+    dp.DS = DS;
+    dp.sdev = sdev;
+    dp.d_pen = a.cot.d_dead_penalty;
+    dp.Tv = Tv;
+    dp.N = N;
+    dp.N64 = N64;
+    dp.routes = R;
+    dp.gp = a.gp;
+    dp.exp_scale = exp_scale;
+    dp.sharp = d.sharpness;
+    if (gl) hipLaunchKernelGGL(bwd_ds_elem_kernel<true>, grid_e, dim3(256), 0, st, dp);
+    else hipLaunchKernelGGL(bwd_ds_elem_kernel<false>, grid_e, dim3(256), 0, st, dp);
+    SRW_TRY(hipGetLastError());
+  }
 
   // the five gradient contractions: bf16 dots, fp32 accumulation
   {
