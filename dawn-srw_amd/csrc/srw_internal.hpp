@@ -107,6 +107,7 @@ struct FinalizeArgs {
   GateParams gp;
   float exp_scale;
   int den_gate;        // den from the gate sum (v4.0.1)
+  int chunk_f32;       // the chunks' sums added in fp32, not rounded to bf16 first (as the generic kernels do)
 };
 hipError_t launch_finalize(const FinalizeArgs& f, hipStream_t s);
 

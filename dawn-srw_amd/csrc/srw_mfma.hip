@@ -2068,7 +2068,8 @@ __device__ __attribute__((always_inline)) inline void diag_maxima(const FinalPar
 // a fixed order, so the result is deterministic (and the same for either
 // VW: each column keeps its order of additions).  Few splits per chunk
 // (large T) use NG = 1, many (decode) NG = 16.
-template <int NG, int VW>
+// F32: the chunks' sums stay fp32 (FinalizeArgs::chunk_f32)
+template <int NG, int VW, bool F32>
 __device__ __attribute__((always_inline)) inline void finalize_body(const FinalParams& p, const int bx, const int by) {
   constexpr int CW = 256 / NG;
   static_assert(VW == 1 || VW == 2 || VW == 4, "one, two or four columns per thread");
@@ -2121,7 +2122,7 @@ __device__ __attribute__((always_inline)) inline void finalize_body(const FinalP
   auto round_v = [](vec_t x) {
     vec_t r;
 #pragma unroll
-    for (int k = 0; k < VW; ++k) r[k] = round_bf16(x[k]);
+    for (int k = 0; k < VW; ++k) r[k] = F32 ? x[k] : round_bf16(x[k]);
     return r;
   };
   if (NG == 1 && p.spc == 1) {
@@ -2210,14 +2211,14 @@ __device__ __attribute__((always_inline)) inline void finalize_body(const FinalP
     }
   }
 }
-template <int NG, int VW = 1>
+template <int NG, int VW = 1, bool F32 = false>
 __global__ __launch_bounds__(256) void srw_finalize_kernel(FinalParams p) {
-  finalize_body<NG, VW>(p, blockIdx.x, blockIdx.y);
+  finalize_body<NG, VW, F32>(p, blockIdx.x, blockIdx.y);
 }
 template <int NG, int VW = 1>
 __global__ __launch_bounds__(256) void srw_finalize_batch_kernel(Batch<FinalParams> b) {
   const int i = batch_index(b.start, b.n, blockIdx.x);
-  finalize_body<NG, VW>(b.p[i], blockIdx.x - b.start[i], blockIdx.y);
+  finalize_body<NG, VW, false>(b.p[i], blockIdx.x - b.start[i], blockIdx.y);
 }
 
 // Few splits per chunk (spc < 16: prefill-sized T): one wave per row, lane l
@@ -2225,7 +2226,7 @@ __global__ __launch_bounds__(256) void srw_finalize_batch_kernel(Batch<FinalPara
 // workgroup.  Each chunk's splits are summed in the order of the NG = 1
 // kernel above (eight accumulators, a fixed tree), so both give the same
 // bits; the per-row partials and diagnostics are reduced across the wave.
-template <int DC>  // d_model / 64
+template <int DC, bool F32>  // d_model / 64
 __device__ __attribute__((always_inline)) inline void finalize_rows_body(const FinalParams& p, const int bid) {
   const int lane = threadIdx.x & 63;
   const int64_t t = static_cast<int64_t>(bid) * 4 + (threadIdx.x >> 6);
@@ -2290,7 +2291,7 @@ __device__ __attribute__((always_inline)) inline void finalize_rows_body(const F
     for (int j = 0; j < DC; ++j) {
       const float* a = acc[j];
       const float sum = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-      raw[j] += round_bf16(sum);                              // bf16 dot output (v41:518)
+      raw[j] += F32 ? sum : round_bf16(sum);                              // bf16 dot output (v41:518)
     }
   }
 #pragma unroll
@@ -2334,14 +2335,14 @@ __device__ __attribute__((always_inline)) inline void finalize_rows_body(const F
   }
 }
 
-template <int DC>
+template <int DC, bool F32 = false>
 __global__ __launch_bounds__(256) void srw_finalize_rows_kernel(FinalParams p) {
-  finalize_rows_body<DC>(p, blockIdx.x);
+  finalize_rows_body<DC, F32>(p, blockIdx.x);
 }
 template <int DC>
 __global__ __launch_bounds__(256) void srw_finalize_rows_batch_kernel(Batch<FinalParams> b) {
   const int i = batch_index(b.start, b.n, blockIdx.x);
-  finalize_rows_body<DC>(b.p[i], blockIdx.x - b.start[i]);
+  finalize_rows_body<DC, false>(b.p[i], blockIdx.x - b.start[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -3406,33 +3407,40 @@ FinalParams final_params_of(const FinalizeArgs& f) {
   return fp;
 }
 
-hipError_t launch_finalize(const FinalizeArgs& f, hipStream_t s) {
+namespace {
+template <bool F32>
+hipError_t launch_finalize_as(const FinalizeArgs& f, hipStream_t s) {
   const FinalParams fp = final_params_of(f);
   const int ng = finalize_groups(f.spc);
   if (ng == 1 && (f.D == 64 || f.D == 128 || f.D == 384)) {
     const dim3 grid_r(static_cast<unsigned>((f.T + 3) / 4));
-    if (f.D == 64) hipLaunchKernelGGL(srw_finalize_rows_kernel<1>, grid_r, dim3(256), 0, s, fp);
-    else if (f.D == 128) hipLaunchKernelGGL(srw_finalize_rows_kernel<2>, grid_r, dim3(256), 0, s, fp);
-    else hipLaunchKernelGGL(srw_finalize_rows_kernel<6>, grid_r, dim3(256), 0, s, fp);
+    if (f.D == 64) hipLaunchKernelGGL((srw_finalize_rows_kernel<1, F32>), grid_r, dim3(256), 0, s, fp);
+    else if (f.D == 128) hipLaunchKernelGGL((srw_finalize_rows_kernel<2, F32>), grid_r, dim3(256), 0, s, fp);
+    else hipLaunchKernelGGL((srw_finalize_rows_kernel<6, F32>), grid_r, dim3(256), 0, s, fp);
     return hipGetLastError();
   }
   const int vw = finalize_width(f.T, f.D, ng);
   const int cols = 256 / ng * vw;  // per workgroup
   const dim3 grid_f(static_cast<unsigned>(f.T), static_cast<unsigned>((f.D + cols - 1) / cols));
   if (vw == 4) {
-    if (ng == 16) hipLaunchKernelGGL((srw_finalize_kernel<16, 4>), grid_f, dim3(256), 0, s, fp);
-    else if (ng == 4) hipLaunchKernelGGL((srw_finalize_kernel<4, 4>), grid_f, dim3(256), 0, s, fp);
-    else hipLaunchKernelGGL((srw_finalize_kernel<1, 4>), grid_f, dim3(256), 0, s, fp);
+    if (ng == 16) hipLaunchKernelGGL((srw_finalize_kernel<16, 4, F32>), grid_f, dim3(256), 0, s, fp);
+    else if (ng == 4) hipLaunchKernelGGL((srw_finalize_kernel<4, 4, F32>), grid_f, dim3(256), 0, s, fp);
+    else hipLaunchKernelGGL((srw_finalize_kernel<1, 4, F32>), grid_f, dim3(256), 0, s, fp);
   } else if (vw == 2) {
-    if (ng == 16) hipLaunchKernelGGL((srw_finalize_kernel<16, 2>), grid_f, dim3(256), 0, s, fp);
-    else if (ng == 4) hipLaunchKernelGGL((srw_finalize_kernel<4, 2>), grid_f, dim3(256), 0, s, fp);
-    else hipLaunchKernelGGL((srw_finalize_kernel<1, 2>), grid_f, dim3(256), 0, s, fp);
+    if (ng == 16) hipLaunchKernelGGL((srw_finalize_kernel<16, 2, F32>), grid_f, dim3(256), 0, s, fp);
+    else if (ng == 4) hipLaunchKernelGGL((srw_finalize_kernel<4, 2, F32>), grid_f, dim3(256), 0, s, fp);
+    else hipLaunchKernelGGL((srw_finalize_kernel<1, 2, F32>), grid_f, dim3(256), 0, s, fp);
   } else {
-    if (ng == 16) hipLaunchKernelGGL(srw_finalize_kernel<16>, grid_f, dim3(256), 0, s, fp);
-    else if (ng == 4) hipLaunchKernelGGL(srw_finalize_kernel<4>, grid_f, dim3(256), 0, s, fp);
-    else hipLaunchKernelGGL(srw_finalize_kernel<1>, grid_f, dim3(256), 0, s, fp);
+    if (ng == 16) hipLaunchKernelGGL((srw_finalize_kernel<16, 1, F32>), grid_f, dim3(256), 0, s, fp);
+    else if (ng == 4) hipLaunchKernelGGL((srw_finalize_kernel<4, 1, F32>), grid_f, dim3(256), 0, s, fp);
+    else hipLaunchKernelGGL((srw_finalize_kernel<1, 1, F32>), grid_f, dim3(256), 0, s, fp);
   }
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_finalize(const FinalizeArgs& f, hipStream_t s) {
+  return f.chunk_f32 ? launch_finalize_as<true>(f, s) : launch_finalize_as<false>(f, s);
 }
 
 // The batch twin of a prefill main kernel (non-diagnostic instantiations).

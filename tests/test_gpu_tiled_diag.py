@@ -81,6 +81,26 @@ def test_tiled_diagnostics_match_generic(pkg, dev, case):
     assert torch.allclose(f["unit_diag"][:, 1], g["unit_diag"][:, 1], rtol=2e-3, atol=1e-6)
 
 
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "T{}D{}dr{}N{}R{}c{}".format(*c[:6]))
+def test_tiled_diagnostics_round_out_once(pkg, dev, case):
+    """out is as exact as the scalar kernels': the chunks' sums are not rounded
+    to bf16 before the division.  What is left against them is the order of
+    the fp32 sums, which moves an element to the neighbouring bf16 value now
+    and then, and gates of scores that round the other way; a second rounding
+    of every element is 2^-9 / sqrt(3) rms or more over a binade, 1.1e-3."""
+    print(f"[gpu] tiled diagnostics, rounding {case}", flush=True)
+    _, args, cs = _call(pkg, dev, case)
+    outs = []
+    for general in (False, True):
+        plan = pkg.SrwPlan(*args, chunk_size=cs, diag=True)
+        if general:
+            plan._desc.flags |= pkg._capi.SRW_FLAG_NO_FAST
+        plan.launch()
+        outs.append(plan.out.float().cpu())
+        assert plan.path == ("generic" if general else "tiled_bf16")
+    assert rel_fro(outs[0], outs[1]) <= 1e-3
+
+
 def test_diagnostics_kept_on_generic(pkg, dev):
     """What the tiled diagnostics do not cover keeps the scalar kernels: gate
     constants under which gate and intensity are not non-decreasing in the
