@@ -58,7 +58,7 @@ int choose(const srw_desc_t& d, bool h_is_x) {
     if (srw::mfma_supports(d, h_is_x)) return 1;
     if (srw::tiled_supports(d)) return 2;
     // diagnostics at the widths the fused kernels do not take: a training step
-    // at T = 2 036, N = 20 011, d_model 1 024, d_route 256 takes 1.88 ms, on
+    // at T = 2 036, N = 20 011, d_model 1 024, d_route 256 takes 1.33 ms, on
     // the generic kernels 58.3
     if (srw::tiled_diag_supports(d)) return 2;
     if (srw::tiled_f32_supports(d)) return 3;
