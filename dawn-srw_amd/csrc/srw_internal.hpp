@@ -172,38 +172,6 @@ bool tiled_f32_supports(const srw_desc_t& d);
 size_t tiled_f32_workspace_bytes(const srw_desc_t& d);
 hipError_t tiled_f32_forward(const LaunchArgs& a);
 
-// The fp32 family's GEMMs with each operand as two fp16 numbers, see
-// srw_split_f32.hip.  A score / gate tile is 128 units x 128 tokens; moments
-// and sums are per unit tile.
-struct SplitArgs {
-  int* flags;               // [0] a token row, [1] a pool row that the split does not take
-  unsigned* rmax;           // (flags + 2) largest |r_n| / (scale of w_n) as float bits; smallest, from 0x7f800000 down
-  const char *x, *h, *e, *r, *wt;  // split rows: [T, D], [Tv, dr] (or x), [N, dr], [N, D], [D, N64]
-  const float *ix, *ih, *ie, *irw; // inverse scales (irw: of r and w together; ie, irw [N64])
-  const float* xnorm;       // [T] |x|
-  float* sp;                // [Tv] scale of P's rows
-  float* S;                 // [Tv, N64] scores, then split P
-  float *mom, *smax;        // [CT][Tv][2], [CT][Tv]
-  const float *tau, *sstd;  // [Tv]; sstd: the v4.0.1 gate
-  float* tok_part;          // [CT][Tv][4]
-  uint32_t* mask32;
-  int64_t mask_words32;
-  float* G;                 // [Tv, N] or null
-  float* out_part;          // [WS][Tv][D]
-  int64_t Tv, N, N64, D, dr;
-  int routes, RT, CT, centred;
-  int WRT, WDT, WS, nkb, W8;
-  GateParams gp;
-};
-struct SplitSources {  // fp32 inputs and the scratch of the pool's scales
-  const float *x, *h, *e, *r, *w;
-  float *ir, *rnorm, *iw;   // [N] each
-};
-hipError_t split_prepare(const SplitArgs& a, const SplitSources& q, bool pool, hipStream_t s);
-hipError_t split_stats(const SplitArgs& a, hipStream_t s);
-hipError_t split_gate(const SplitArgs& a, hipStream_t s);  // rows' scales, then the gate kernel
-hipError_t split_write(const SplitArgs& a, bool w192, hipStream_t s);
-
 // MFMA kernels (bf16 / f32 matrix cores), see srw_mfma.hip.
 size_t mfma_workspace_bytes(const srw_desc_t& d);
 // h_is_x: h aliases x (d_route == d_model, one route), which some shapes need

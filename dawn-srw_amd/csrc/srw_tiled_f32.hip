@@ -190,9 +190,8 @@ __device__ inline bool ftile_of(int nrow, int ncol, int& rt, int& ct) {
 // pack: W [N, D] -> W^T [D, N64], zero for units >= N
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void pack_wt_f32_kernel(const float* __restrict__ W, float* __restrict__ WT,
-                                                          int64_t N, int64_t N64, int D, const int* flags) {
+                                                          int64_t N, int64_t N64, int D) {
   __shared__ float tile[64][65];
-  if (flags && !(flags[0] | flags[1])) return;
   const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 64;
   const int d0 = blockIdx.y * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
@@ -220,12 +219,7 @@ struct FStatsParams {
   int64_t Tv, N, N64, dr;
   int RT, CT;    // token tiles, unit tiles
   int centred;   // second moments about the 128 units' own mean (merged by srw_tau_kernel's kTauChan)
-  const int* flags;  // behind the split kernels: run only where one is set; or null
 };
-
-// Behind the split kernels (srw_split_f32.hip) the fp32 ones run only where a
-// flag is set.
-__device__ inline bool not_needed(const int* flags) { return flags && !(flags[0] | flags[1]); }
 
 // A workgroup takes 256 units x 64 MJ tokens (2 x 2 waves of 128 units x
 // 32 MJ tokens).  The launches use MJ = 1: 80 KB of LDS and ~180 registers a
@@ -236,7 +230,6 @@ __device__ inline bool not_needed(const int* flags) { return flags && !(flags[0]
 template <int MJ>
 __global__ __launch_bounds__(kFThreads, 1) void f32_stats_kernel(FStatsParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  if (not_needed(p.flags)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wa = wave >> 1, wb = wave & 1, u = lane & 31, h = lane >> 5;
@@ -324,7 +317,6 @@ struct FGateParams {
   int64_t Tv, N, N64, D;
   int routes, RT, CT;  // token tiles, unit tiles
   GateParams gp;
-  const int* flags;
 };
 
 // tiles as f32_stats_kernel's.  GL: the v4.0.1 gate of _srw_inference
@@ -334,7 +326,6 @@ struct FGateParams {
 template <int MJ, bool GL>
 __global__ __launch_bounds__(kFThreads, 1) void f32_gate_kernel(FGateParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  if (not_needed(p.flags)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wa = wave >> 1, wb = wave & 1, u = lane & 31, h = lane >> 5;
@@ -429,7 +420,6 @@ struct FWriteParams {
   int64_t Tv, N64, D;
   int S, RT, DT, nkb;  // RT, DT: token and column tiles of this kernel's tile shape; nkb: 32-unit k blocks
   int W8;              // (token tile, split) pairs per XCD
-  const int* flags;
 };
 
 // A workgroup computes a (32 GA tokens) x (32 GB columns) tile of one split's
@@ -444,7 +434,6 @@ __global__ __launch_bounds__(kFThreads, 1) void f32_write_kernel(FWriteParams p)
   static_assert(GA % MI == 0 && GB % MJ == 0 && (GA / MI) * (GB / MJ) == kFThreads / 64,
                 "one accumulator block per wave");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  if (not_needed(p.flags)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int WB = GB / MJ;
@@ -582,12 +571,10 @@ FGeo fgeo(const srw_desc_t& d) {
 }
 
 struct FLayout {
-  size_t wt, P, mom, tau, out_part, tok_part, rn, wn, sstd;
-  size_t flags, sx, sh, se, sr, swt, ix, ih, ie, ir, rnorm, iw, irw, xnorm, sp, smax;  // the split kernels'
-  size_t total;
+  size_t wt, P, mom, tau, out_part, tok_part, rn, wn, sstd, total;
 };
 
-FLayout flayout(const srw_desc_t& d, const FGeo& g, bool split) {
+FLayout flayout(const srw_desc_t& d, const FGeo& g) {
   FLayout l{};
   size_t off = 0;
   l.wt = off;
@@ -609,45 +596,8 @@ FLayout flayout(const srw_desc_t& d, const FGeo& g, bool split) {
     l.sstd = l.wn + fal256(d.n_units * d.d_model * 4);
     off = l.sstd + fal256(g.Tv * 4);
   }
-  if (split) {
-    auto take = [&](int64_t bytes) {
-      const size_t at = off;
-      off += fal256(bytes);
-      return at;
-    };
-    const int64_t D = d.d_model, dr = d.d_route;
-    l.flags = take(4 * 4);
-    l.sx = take(d.T * D * 4);
-    l.sh = take(g.Tv * dr * 4);
-    l.se = take(g.N * dr * 4);
-    l.sr = take(g.N * D * 4);
-    l.swt = take(D * g.N64 * 4);
-    l.ix = take(d.T * 4);
-    l.ih = take(g.Tv * 4);
-    l.ie = take(g.N64 * 4);
-    l.ir = take(g.N * 4);
-    l.rnorm = take(g.N * 4);
-    l.iw = take(g.N * 4);
-    l.irw = take(g.N64 * 4);
-    l.xnorm = take(d.T * 4);
-    l.sp = take(g.Tv * 4);
-    l.smax = take(static_cast<int64_t>(2 * g.CT) * g.Tv * 4);
-  }
   l.total = off;
   return l;
-}
-
-// The split kernels (srw_split_f32.hip): widths from 128 on, where two fp16
-// numbers are the more exact form; token counts that pay for splitting the
-// pool's rows (srw_inference at d 384, split against fp32, us: N = 25 200: T =
-// 128 about even, 256 234 / 259, 512 267 / 386, 2 048 579 / 1 192; N = 2 600:
-// T = 256 98 / 125, 2 048 125 / 194); and never a call that srw_forward_noalloc's scratch holds
-// without the split rows but not with them (its results equal srw_forward's
-// bit for bit).
-constexpr int64_t kSplitMinRows = 256;
-bool split_applies(const srw_desc_t& d, const FGeo& g) {
-  if (d.d_model < 128 || d.d_route < 128 || g.Tv < kSplitMinRows) return false;
-  return flayout(d, g, false).total > SRW_NOALLOC_SCRATCH_BYTES || flayout(d, g, true).total <= SRW_NOALLOC_SCRATCH_BYTES;
 }
 
 }  // namespace
@@ -664,19 +614,13 @@ bool tiled_f32_supports(const srw_desc_t& d) {
   return true;
 }
 
-size_t tiled_f32_workspace_bytes(const srw_desc_t& d) {
-  const FGeo g = fgeo(d);
-  return flayout(d, g, split_applies(d, g)).total;
-}
+size_t tiled_f32_workspace_bytes(const srw_desc_t& d) { return flayout(d, fgeo(d)).total; }
 
 hipError_t tiled_f32_forward(const LaunchArgs& a) {
   const srw_desc_t& d = a.d;
   const FGeo g = fgeo(d);
-  const bool split = split_applies(d, g);
-  const FLayout l = flayout(d, g, split);
+  const FLayout l = flayout(d, g);
   if (a.ws_bytes < l.total) return hipErrorInvalidValue;
-  auto at = [&](size_t off) { return reinterpret_cast<float*>(a.ws + off); };
-  const int* flags = split ? reinterpret_cast<const int*>(a.ws + l.flags) : nullptr;
   float* wt = reinterpret_cast<float*>(a.ws + l.wt);
   float* P = reinterpret_cast<float*>(a.ws + l.P);
   float* mom = reinterpret_cast<float*>(a.ws + l.mom);
@@ -708,51 +652,10 @@ hipError_t tiled_f32_forward(const LaunchArgs& a) {
     read_rows = rn;
     write_rows = wn;
   }
-  SplitArgs sa{};
-  if (split) {
-    sa.flags = reinterpret_cast<int*>(a.ws + l.flags);
-    sa.rmax = reinterpret_cast<unsigned*>(a.ws + l.flags) + 2;
-    sa.x = a.ws + l.sx;
-    sa.h = a.in.h == a.in.x ? sa.x : a.ws + l.sh;
-    sa.e = a.ws + l.se;
-    sa.r = a.ws + l.sr;
-    sa.wt = a.ws + l.swt;
-    sa.ix = at(l.ix);
-    sa.ih = a.in.h == a.in.x ? sa.ix : at(l.ih);
-    sa.ie = at(l.ie);
-    sa.irw = at(l.irw);
-    sa.xnorm = at(l.xnorm);
-    sa.sp = at(l.sp);
-    sa.S = P;
-    sa.mom = mom;
-    sa.smax = at(l.smax);
-    sa.tau = tau;
-    sa.sstd = gl ? at(l.sstd) : nullptr;
-    sa.tok_part = tok_part;
-    sa.mask32 = reinterpret_cast<uint32_t*>(a.o.pass_mask);
-    sa.mask_words32 = 2 * a.words;
-    sa.G = (d.flags & SRW_FLAG_GATE_OUT) ? a.o.gate : nullptr;
-    sa.out_part = out_part;
-    sa.Tv = g.Tv;
-    sa.N = g.N;
-    sa.N64 = g.N64;
-    sa.D = D;
-    sa.dr = d.d_route;
-    sa.routes = d.n_routes;
-    sa.RT = static_cast<int>((g.Tv + 127) / 128);
-    sa.CT = 2 * g.CT;  // the fp32 kernels' slices of 128 units
-    sa.centred = d.stats_mode == SRW_STATS_CENTERED;
-    sa.WRT = g.WRT;
-    sa.WDT = g.DT;
-    sa.WS = g.S;
-    sa.nkb = g.nkb;
-    sa.W8 = g.W8;
-    sa.gp = a.gp;
-    const SplitSources q{static_cast<const float*>(a.in.x), static_cast<const float*>(a.in.h),
-                         static_cast<const float*>(a.in.emb), read_rows, write_rows,
-                         at(l.ir), at(l.rnorm), at(l.iw)};
-    if ((e = split_prepare(sa, q, !(d.flags & SRW_FLAG_POOL_CACHED), a.stream)) != hipSuccess) return e;
-    if ((e = split_stats(sa, a.stream)) != hipSuccess) return e;
+  if (!(d.flags & SRW_FLAG_POOL_CACHED)) {
+    const dim3 grid_p(static_cast<unsigned>(g.N64 / 64), static_cast<unsigned>((D + 63) / 64));
+    hipLaunchKernelGGL(pack_wt_f32_kernel, grid_p, dim3(256), 0, a.stream, write_rows, wt, g.N, g.N64, D);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   // score and gate kernels: 256-unit x 64-token tiles, two stages of 256 + 64 operand rows
   const dim3 grid_q(static_cast<unsigned>(8 * g.RTq * ((g.CT + 7) / 8)));
@@ -769,7 +672,6 @@ hipError_t tiled_f32_forward(const LaunchArgs& a) {
   sp.centred = d.stats_mode == SRW_STATS_CENTERED;
   sp.RT = g.RTq;
   sp.CT = g.CT;
-  sp.flags = flags;
   hipLaunchKernelGGL(f32_stats_kernel<1>, grid_q, dim3(kFThreads), kLdsQ, a.stream, sp);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   // tau per row from the 2 CT partials of 128 units (centred: merged by
@@ -780,16 +682,7 @@ hipError_t tiled_f32_forward(const LaunchArgs& a) {
       hipSuccess)
     return e;
 
-  if (split && (e = split_gate(sa, a.stream)) != hipSuccess) return e;
-  // W^T: behind the split kernels only where a flag is set (split_gate sets the
-  // last one), of a cached pool too: the flag may be this call's tokens'
-  if (split || !(d.flags & SRW_FLAG_POOL_CACHED)) {
-    const dim3 grid_p(static_cast<unsigned>(g.N64 / 64), static_cast<unsigned>((D + 63) / 64));
-    hipLaunchKernelGGL(pack_wt_f32_kernel, grid_p, dim3(256), 0, a.stream, write_rows, wt, g.N, g.N64, D, flags);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
   FGateParams gp{};
-  gp.flags = flags;
   gp.x = static_cast<const float*>(a.in.x);
   gp.read = read_rows;
   gp.sstd = sstd;
@@ -805,19 +698,17 @@ hipError_t tiled_f32_forward(const LaunchArgs& a) {
   gp.D = D;
   gp.routes = d.n_routes;
   gp.gp = a.gp;
-  if (!split) dominant_kernel_begin(a.stream);
+  dominant_kernel_begin(a.stream);
   gp.RT = g.RTq;
   gp.CT = g.CT;
   if (gl)
     hipLaunchKernelGGL((f32_gate_kernel<1, true>), grid_q, dim3(kFThreads), kLdsQ, a.stream, gp);
   else
     hipLaunchKernelGGL((f32_gate_kernel<1, false>), grid_q, dim3(kFThreads), kLdsQ, a.stream, gp);
-  if (!split) dominant_kernel_end(a.stream);
+  dominant_kernel_end(a.stream);
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
-  if (split && (e = split_write(sa, g.w192, a.stream)) != hipSuccess) return e;
   FWriteParams wp{};
-  wp.flags = flags;
   wp.P = P;
   wp.wt = wt;
   wp.out_part = out_part;
