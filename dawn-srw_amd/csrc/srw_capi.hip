@@ -47,8 +47,9 @@ srw_status_t validate(const srw_desc_t* d) {
 
 // Which family serves this descriptor: 1 = fused MFMA, 2 = tiled GEMMs,
 // 3 = fp32 tiled GEMMs, 0 = generic, -1 = none.  h_is_x: h aliases x (known to srw_forward from
-// the pointers).
-int choose(const srw_desc_t& d, bool h_is_x) {
+// the pointers).  tiled_diag false: without the diagnostics on the tiled
+// family, whose place the generic kernels take.
+int choose(const srw_desc_t& d, bool h_is_x, bool tiled_diag = true) {
   const bool force_generic = (d.flags & (SRW_FLAG_EMULATE | SRW_FLAG_NO_FAST)) != 0;
   if (!force_generic && (d.flags & SRW_FLAG_GATE_OUT)) {  // the dense gate from the tiled gate epilogue
     if (srw::tiled_supports(d)) return 2;
@@ -60,7 +61,7 @@ int choose(const srw_desc_t& d, bool h_is_x) {
     // diagnostics at the widths the fused kernels do not take: a training step
     // at T = 2 036, N = 20 011, d_model 1 024, d_route 256 takes 1.33 ms, on
     // the generic kernels 58.3
-    if (srw::tiled_diag_supports(d)) return 2;
+    if (tiled_diag && srw::tiled_diag_supports(d)) return 2;
     if (srw::tiled_f32_supports(d)) return 3;
   }
   if (d.stats_mode == SRW_STATS_GRAM) return -1;  // only the MFMA family implements it
@@ -111,6 +112,24 @@ size_t bytes_of(int which, const srw_desc_t& d) {
   if (which == 2) return srw::tiled_workspace_bytes(d);
   if (which == 3) return srw::tiled_f32_workspace_bytes(d);
   return srw::generic_workspace_bytes(d);
+}
+
+// The largest need over the paths a call may take: h aliasing x (possible
+// when d_route == d_model with one route) can select the MFMA family.  False:
+// no family serves the descriptor.
+bool largest_need(const srw_desc_t& d, bool tiled_diag, size_t* bytes) {
+  const bool can_alias = d.n_routes == 1 && d.d_route == d.d_model;
+  const int which = choose(d, false, tiled_diag);
+  const int which_alias = can_alias ? choose(d, true, tiled_diag) : which;
+  if (which < 0 && which_alias < 0) return false;
+  size_t need = 0;
+  for (int w : {which, which_alias}) {
+    if (w < 0 || d.T == 0) continue;  // no tokens: srw_forward needs no workspace
+    const size_t n = align256(bytes_of(w, d));
+    need = n > need ? n : need;
+  }
+  *bytes = need;
+  return true;
 }
 
 }  // namespace
@@ -170,20 +189,7 @@ srw_status_t srw_workspace_size(const srw_desc_t* d, size_t* bytes) {
   srw_status_t st = validate(d);
   if (st != SRW_OK) return st;
   if (!bytes) return SRW_EINVAL;
-  // the largest need over the paths a call may take: h aliasing x (possible
-  // when d_route == d_model with one route) can select the MFMA family
-  const bool can_alias = d->n_routes == 1 && d->d_route == d->d_model;
-  const int which = choose(*d, false);
-  const int which_alias = can_alias ? choose(*d, true) : which;
-  if (which < 0 && which_alias < 0) return SRW_EUNSUPPORTED;
-  size_t need = 0;
-  for (int w : {which, which_alias}) {
-    if (w < 0 || d->T == 0) continue;  // no tokens: srw_forward needs no workspace
-    const size_t n = align256(bytes_of(w, *d));
-    need = n > need ? n : need;
-  }
-  *bytes = need;
-  return SRW_OK;
+  return largest_need(*d, true, bytes) ? SRW_OK : SRW_EUNSUPPORTED;
 }
 
 }  // extern "C"
@@ -279,12 +285,16 @@ srw_status_t srw_forward_noalloc(const srw_desc_t* d, const srw_tensors_t* in, c
   size_t need = 0;
   if ((st = srw_workspace_size(d, &need)) != SRW_OK) return st;
   srw_desc_t small;
-  if (need > SRW_NOALLOC_SCRATCH_BYTES && (d->flags & SRW_FLAG_DIAG) && in && choose(*d, in->h == in->x) == 2) {
-    // diagnostics on the tiled family do not fit; the generic kernels need no workspace
-    small = *d;
-    small.flags |= SRW_FLAG_NO_FAST;
-    d = &small;
-    if ((st = srw_workspace_size(d, &need)) != SRW_OK) return st;
+  if (need > SRW_NOALLOC_SCRATCH_BYTES && (d->flags & SRW_FLAG_DIAG)) {
+    // without the diagnostics on the tiled family, which are not this call's
+    // where h == x selects the MFMA family and where they do not fit give way
+    // to the generic kernels, which need no workspace
+    (void)largest_need(*d, false, &need);
+    if (in && choose(*d, in->h != nullptr && in->h == in->x) == 2) {
+      small = *d;
+      small.flags |= SRW_FLAG_NO_FAST;
+      d = &small;
+    }
   }
   if (need > SRW_NOALLOC_SCRATCH_BYTES) return SRW_ESCRATCH;
   void* ws = nullptr;

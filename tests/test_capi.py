@@ -203,6 +203,23 @@ def test_noalloc_refusals_before_any_launch(C):
     assert lib.srw_forward_noalloc(ctypes.byref(d), ctypes.byref(t), ctypes.byref(o), None) == C.SRW_OK
 
 
+@pytest.mark.parametrize("T", [1024, 2048])
+def test_noalloc_takes_diagnostics_of_h_equal_x(C, T):
+    """With diagnostics at d_route == d_model, a call with h == x runs on the
+    fused kernels, whose workspace the scratch holds here; the tiled family,
+    which a call with another h would take, does not fit and is not asked.
+    (A missing emb ends the call behind the scratch check.)"""
+    d = C.desc_init()
+    d.T, d.d_model, d.d_route, d.n_units, d.chunk_size, d.flags = T, 384, 384, 2600, 2600, C.SRW_FLAG_DIAG
+    assert C.workspace_size(d) > C.NOALLOC_SCRATCH_BYTES
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.cast(buf, ctypes.c_void_p)
+    tens = C.SrwTensors(p, p, None, p, p, p)
+    outs = C.SrwOutputs(out=p)
+    st = C.load_library().srw_forward_noalloc(ctypes.byref(d), ctypes.byref(tens), ctypes.byref(outs), None)
+    assert st not in (C.SRW_ESCRATCH, C.SRW_EWORKSPACE, C.SRW_OK)
+
+
 def test_status_strings(C):
     lib = C.load_library()
     for s in range(6):
