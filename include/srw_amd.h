@@ -276,12 +276,17 @@ srw_status_t srw_forward(const srw_desc_t* desc, const srw_tensors_t* in,
  * SRW_NOALLOC_SCRATCH_BYTES inside the library, one per GPU, held from the
  * library's first use on that GPU until the process ends; its device address
  * is looked up once per device.  The same kernels run as in srw_forward, so
- * the results are equal bit for bit.  Limits: a call whose
- * srw_workspace_size exceeds the scratch returns SRW_ESCRATCH with nothing
- * launched (64 MiB holds every decode-sized call of the 40M pools up to 128
- * rows; prefill-sized calls need srw_forward); SRW_FLAG_POOL_CACHED is
- * refused (SRW_EINVAL), since the scratch keeps whatever the last call on that
- * GPU left in it.  All calls on one GPU share its scratch: calls that overlap
+ * the results are equal bit for bit, but for one kind of call: SRW_FLAG_DIAG at
+ * widths whose diagnostics srw_forward takes on the tiled family ("tiled_bf16")
+ * runs on the generic kernels here where the tiled workspace exceeds the
+ * scratch, with the results of srw_forward under SRW_FLAG_NO_FAST (unit_diag's
+ * sums, which those kernels add up in no fixed order, aside).  Limits: any
+ * other call whose srw_workspace_size exceeds the scratch returns SRW_ESCRATCH
+ * with nothing launched (64 MiB holds every decode-sized call of the 40M pools
+ * up to 128 rows; prefill-sized calls need srw_forward; with SRW_FLAG_DIAG the
+ * size without the tiled family decides); SRW_FLAG_POOL_CACHED is refused
+ * (SRW_EINVAL), since the scratch keeps whatever the last call on that GPU
+ * left in it.  All calls on one GPU share its scratch: calls that overlap
  * on one GPU (two streams, two threads) race -- serialise them. */
 #define SRW_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
 srw_status_t srw_forward_noalloc(const srw_desc_t* desc, const srw_tensors_t* in,
