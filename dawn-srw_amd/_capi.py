@@ -53,7 +53,7 @@ UDIAG = ("score_sum", "gate_max")
 # Every symbol include/srw_amd.h declares.
 EXPORTED_SYMBOLS = (
     "srw_abi_version", "srw_status_string", "srw_desc_init",
-    "srw_workspace_size", "srw_forward", "srw_last_path",
+    "srw_workspace_size", "srw_workspace_size_for", "srw_forward", "srw_last_path",
     "srw_set_kernel_events", "srw_backward_workspace_size", "srw_backward",
     "srw_workspace_size_batch", "srw_forward_batch", "srw_forward_noalloc",
     "srw_diag_summary", "srw_cast_bf16", "srw_dawn_decode_step",
@@ -163,6 +163,9 @@ def load_library() -> ctypes.CDLL:
         lib.srw_desc_init.argtypes = [ctypes.POINTER(SrwDesc)]
         lib.srw_workspace_size.restype = ctypes.c_int
         lib.srw_workspace_size.argtypes = [ctypes.POINTER(SrwDesc), ctypes.POINTER(ctypes.c_size_t)]
+        lib.srw_workspace_size_for.restype = ctypes.c_int
+        lib.srw_workspace_size_for.argtypes = [ctypes.POINTER(SrwDesc), ctypes.POINTER(SrwTensors),
+                                               ctypes.POINTER(ctypes.c_size_t)]
         lib.srw_forward.restype = ctypes.c_int
         lib.srw_forward.argtypes = [
             ctypes.POINTER(SrwDesc), ctypes.POINTER(SrwTensors), ctypes.POINTER(SrwOutputs),
@@ -220,6 +223,13 @@ def desc_init() -> SrwDesc:
 def workspace_size(desc: SrwDesc) -> int:
     n = ctypes.c_size_t(0)
     check(load_library().srw_workspace_size(ctypes.byref(desc), ctypes.byref(n)))
+    return int(n.value)
+
+
+def workspace_size_for(desc: SrwDesc, tens: SrwTensors) -> int:
+    """srw_workspace_size_for: of the call with these tensors."""
+    n = ctypes.c_size_t(0)
+    check(load_library().srw_workspace_size_for(ctypes.byref(desc), ctypes.byref(tens), ctypes.byref(n)))
     return int(n.value)
 
 

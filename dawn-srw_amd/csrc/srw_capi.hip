@@ -192,6 +192,16 @@ srw_status_t srw_workspace_size(const srw_desc_t* d, size_t* bytes) {
   return largest_need(*d, true, bytes) ? SRW_OK : SRW_EUNSUPPORTED;
 }
 
+srw_status_t srw_workspace_size_for(const srw_desc_t* d, const srw_tensors_t* in, size_t* bytes) {
+  srw_status_t st = validate(d);
+  if (st != SRW_OK) return st;
+  if (!in || !bytes) return SRW_EINVAL;
+  const int w = choose(*d, in->h != nullptr && in->h == in->x);
+  if (w < 0) return SRW_EUNSUPPORTED;
+  *bytes = d->T == 0 ? 0 : align256(bytes_of(w, *d));
+  return SRW_OK;
+}
+
 }  // extern "C"
 
 namespace {
@@ -468,7 +478,7 @@ srw_status_t srw_dawn_decode_step(const srw_dawn_step_t* s, void* stream) {
   srw_status_t st = srw_workspace_size_batch(2, s->descs, &need);
   if (st != SRW_OK) return st;
   if (need > 0 && (!s->ws_qkv || s->ws_qkv_bytes < need)) return SRW_EWORKSPACE;
-  if ((st = srw_workspace_size(&s->descs[2], &need)) != SRW_OK) return st;
+  if ((st = srw_workspace_size_for(&s->descs[2], &s->tensors[2], &need)) != SRW_OK) return st;
   if (need > 0 && (!s->ws_know || s->ws_know_bytes < need)) return SRW_EWORKSPACE;
   (void)hipGetLastError();
   return srw::dawn_decode_step(*s, static_cast<hipStream_t>(stream)) == hipSuccess ? SRW_OK : SRW_EHIP;

@@ -127,15 +127,15 @@ class SrwPlan:
                           if diag else None)
         self.gate = (torch.empty((T, R, N), dtype=torch.float32, device=dev)
                      if want_gate else None)
-        self.ws_bytes = C.workspace_size(desc)
+        self._tens = C.SrwTensors(_ptr(x), _ptr(x if h_is_x else h), _ptr(emb),
+                                  _ptr(tau_offset), _ptr(read), _ptr(write))
+        self.ws_bytes = C.workspace_size_for(desc, self._tens)
         self.workspace = torch.empty(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
 
         self.inputs = (x, h, emb, tau_offset, read, write)
         self.device = dev
         self.shape = dict(T=T, D=D, dr=dr, N=N, R=R)
         self._desc = desc
-        self._tens = C.SrwTensors(_ptr(x), _ptr(x if h_is_x else h), _ptr(emb),
-                                  _ptr(tau_offset), _ptr(read), _ptr(write))
         self._outs = C.SrwOutputs(_ptr(self.out), _ptr(self.gate_sum), _ptr(self.den),
                                   _ptr(self.n_active), _ptr(self.pass_mask),
                                   _ptr(self.token_diag), _ptr(self.unit_diag), _ptr(self.gate))

@@ -263,6 +263,11 @@ srw_status_t srw_desc_init(srw_desc_t* desc);
  * d_model and one route, passing h == x can select a different family). */
 srw_status_t srw_workspace_size(const srw_desc_t* desc, size_t* bytes);
 
+/* The workspace of the call with these tensors, of which only whether h == x
+ * is read: never more than srw_workspace_size, and less where the family of
+ * another h is the larger one (diagnostics at d_route == d_model). */
+srw_status_t srw_workspace_size_for(const srw_desc_t* desc, const srw_tensors_t* in, size_t* bytes);
+
 /* Enqueue one SRW layer forward on `stream`.  Replaces fused_gate_srw /
  * fused_gate_srw_paired / _srw_inference (see the table at the top). */
 srw_status_t srw_forward(const srw_desc_t* desc, const srw_tensors_t* in,
@@ -407,7 +412,7 @@ typedef struct srw_dawn_step {
   const srw_outputs_t* outs;    /* host, [3] */
   void* ws_qkv;                 /* srw_workspace_size_batch(2, descs) bytes */
   size_t ws_qkv_bytes;
-  void* ws_know;                /* srw_workspace_size(&descs[2]) bytes */
+  void* ws_know;                /* srw_workspace_size_for(&descs[2], &tensors[2]) bytes */
   size_t ws_know_bytes;
   const char** path_qkv;        /* host: srw_last_path() after the QK and V calls; or NULL */
 } srw_dawn_step_t;

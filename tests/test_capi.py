@@ -220,6 +220,28 @@ def test_noalloc_takes_diagnostics_of_h_equal_x(C, T):
     assert st not in (C.SRW_ESCRATCH, C.SRW_EWORKSPACE, C.SRW_OK)
 
 
+def test_workspace_of_the_call(C):
+    """srw_workspace_size_for: the family that the tensors select; the larger
+    of h == x and another h is srw_workspace_size.  A diagnostic Know call with
+    h == x needs nothing of the tiled family's."""
+    p, q = ctypes.c_void_p(4096), ctypes.c_void_p(8192)
+    same, other = C.SrwTensors(p, p, p, p, p, p), C.SrwTensors(p, q, p, p, p, p)
+    for kw in (dict(flags=C.SRW_FLAG_DIAG), dict(), dict(d_route=128), dict(T=0), dict(dtype=C.SRW_F32)):
+        d = _desc(C, **{**dict(T=4096, d_model=384, d_route=384, n_units=25200, chunk_size=12600), **kw})
+        a, b = C.workspace_size_for(d, same), C.workspace_size_for(d, other)
+        assert max(a, b) == C.workspace_size(d) if d.d_route == d.d_model else b == C.workspace_size(d), kw
+    d = _desc(C, T=4096, d_model=384, d_route=384, n_units=25200, chunk_size=12600, flags=C.SRW_FLAG_DIAG)
+    assert C.workspace_size_for(d, same) < C.workspace_size_for(d, other)
+    d.flags |= C.SRW_FLAG_NO_FAST
+    assert C.workspace_size_for(d, other) == 0
+    n = ctypes.c_size_t(0)
+    lib = C.load_library()
+    assert lib.srw_workspace_size_for(ctypes.byref(d), None, ctypes.byref(n)) == C.SRW_EINVAL
+    assert lib.srw_workspace_size_for(ctypes.byref(d), ctypes.byref(same), None) == C.SRW_EINVAL
+    d.n_routes = 3
+    assert lib.srw_workspace_size_for(ctypes.byref(d), ctypes.byref(same), ctypes.byref(n)) == C.SRW_EINVAL
+
+
 def test_status_strings(C):
     lib = C.load_library()
     for s in range(6):

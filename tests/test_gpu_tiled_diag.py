@@ -145,3 +145,16 @@ def test_noalloc_diagnostics_beyond_the_scratch(pkg, dev):
     # eight scores a unit, in any order: seven additions of at most the sum of their sizes
     inp_s = (args[1][:, 0].float() @ args[2].float().T).abs().sum(0)
     assert ((plan.unit_diag[:, 0] - want["unit_diag"][:, 0]).abs() <= 7 * 2.0 ** -24 * 1.01 * inp_s).all()
+
+
+def test_plan_with_h_equal_x_holds_its_own_workspace(pkg, dev):
+    """With diagnostics at d_route == d_model, h == x runs on the fused kernels:
+    its plan does not allocate the tiled family's larger workspace."""
+    _, args, cs = _call(pkg, dev, (2048, 384, 384, 2600, 1, 2600, 7))
+    print("[gpu] diagnostics plan, h == x", flush=True)
+    same = pkg.SrwPlan(args[0], args[0], *args[2:], chunk_size=cs, diag=True)
+    other = pkg.SrwPlan(*args, chunk_size=cs, diag=True)
+    for p in (same, other):
+        p.launch()
+    assert same.path.startswith("mfma") and other.path == "tiled_bf16"
+    assert same.ws_bytes < other.ws_bytes == pkg._capi.workspace_size(same._desc)
