@@ -45,6 +45,21 @@ srw_status_t validate(const srw_desc_t* d) {
   return SRW_OK;
 }
 
+// Diagnostics on the tiled family pay from a pool size on: seven launches of
+// ~11 us against one generic kernel whose time goes with the units, their
+// widths and the rows past two per CU.  Tiled / generic in us at (d_model,
+// d_route) = (192, 64), (384, 384), (1024, 256):
+//   16 rows:   N = 33 79/25 89/44 98/59;    128 79/51 88/79 96/111;  256 70/86 80/129 87/186
+//   512 rows:  N = 33 107/44 116/59 126/77; 128 107/69 116/91 126/130; 256 98/105 108/146 119/201
+//   1024 rows: N = 33 109/69 117/82 128/97; 128 107/103 117/125 135/154
+//   2048 rows: N = 16 111/77 122/103 137/130; 33 113/124 122/147 138/176
+//   4096 rows: N = 16 120/127 130/157 149/192
+bool tiled_diag_pays(const srw_desc_t& d) {
+  const int64_t rows = d.T * d.n_routes;
+  const int64_t limit = rows <= 512 ? 340000 : rows <= 1024 ? 220000 : rows <= 2048 ? 48000 : 0;
+  return d.n_units * (2 * d.d_model + d.d_route + 1200) > limit;
+}
+
 // Which family serves this descriptor: 1 = fused MFMA, 2 = tiled GEMMs,
 // 3 = fp32 tiled GEMMs, 0 = generic, -1 = none.  h_is_x: h aliases x (known to srw_forward from
 // the pointers).  tiled_diag false: without the diagnostics on the tiled
@@ -61,7 +76,7 @@ int choose(const srw_desc_t& d, bool h_is_x, bool tiled_diag = true) {
     // diagnostics at the widths the fused kernels do not take: a training step
     // at T = 2 036, N = 20 011, d_model 1 024, d_route 256 takes 1.33 ms, on
     // the generic kernels 58.3
-    if (tiled_diag && srw::tiled_diag_supports(d)) return 2;
+    if (tiled_diag && srw::tiled_diag_supports(d) && ((d.flags & SRW_FLAG_TILED) || tiled_diag_pays(d))) return 2;
     if (srw::tiled_f32_supports(d)) return 3;
   }
   if (d.stats_mode == SRW_STATS_GRAM) return -1;  // only the MFMA family implements it

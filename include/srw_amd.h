@@ -126,8 +126,10 @@ typedef enum srw_stats_mode {
                                      in the workspace as bf16) even where a fused kernel
                                      exists; without the flag they serve bf16 shapes the
                                      fused kernels do not (d_model > 384, e.g. 1024 / 1280 /
-                                     2048; both widths multiples of 64).  No counterpart in
-                                     the reference (a kernel-family choice). */
+                                     2048; both widths multiples of 64; with SRW_FLAG_DIAG
+                                     from pools of some hundred units on, with both flags
+                                     from the first).  No counterpart in the reference (a
+                                     kernel-family choice). */
 #define SRW_FLAG_GATE_OUT 0x40u   /* the call passes outputs->gate: the workspace query and
                                      the kernel choice take the tiled matrix-core families
                                      (bf16 d_model / d_route multiples of 64, fp32 multiples

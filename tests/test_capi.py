@@ -242,6 +242,25 @@ def test_workspace_of_the_call(C):
     assert lib.srw_workspace_size_for(ctypes.byref(d), ctypes.byref(same), ctypes.byref(n)) == C.SRW_EINVAL
 
 
+@pytest.mark.parametrize("rows,D,dr,first", [
+    (16, 192, 64, 207), (512, 192, 64, 207), (513, 192, 64, 134), (1024, 1024, 256, 63), (1025, 1024, 256, 14),
+    (2048, 384, 384, 21), (2049, 192, 64, 1)])
+def test_small_pools_keep_their_diagnostics_kernels(C, rows, D, dr, first):
+    """Diagnostics of pools below `first` units run on the generic kernels,
+    which need no workspace; SRW_FLAG_TILED takes them to the tiled family."""
+    p, q = ctypes.c_void_p(4096), ctypes.c_void_p(8192)
+    tens = C.SrwTensors(p, q, p, p, p, p)
+    for routes in (1, 2) if rows % 2 == 0 else (1,):
+        d = _desc(C, T=rows // routes, d_model=D, d_route=dr, n_routes=routes, n_units=first, chunk_size=0,
+                  flags=C.SRW_FLAG_DIAG)
+        assert C.workspace_size_for(d, tens) > 0
+        if first > 1:
+            d.n_units = first - 1
+            assert C.workspace_size_for(d, tens) == 0
+            d.flags |= C.SRW_FLAG_TILED
+            assert C.workspace_size_for(d, tens) > 0
+
+
 def test_status_strings(C):
     lib = C.load_library()
     for s in range(6):

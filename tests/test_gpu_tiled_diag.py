@@ -44,7 +44,7 @@ def test_tiled_diagnostics_match_generic(pkg, dev, case):
     T, D, dr, N, R, _, _ = case
     print(f"[gpu] tiled diagnostics {case}", flush=True)
     inp, args, cs = _call(pkg, dev, case)
-    fast = pkg.srw_forward(*args, chunk_size=cs, diag=True)
+    fast = pkg.srw_forward(*args, chunk_size=cs, diag=True, tiled=True)
     slow = pkg.srw_forward(*args, chunk_size=cs, diag=True, emulate=True)
     torch.cuda.synchronize()
     assert fast["path"] == "tiled_bf16" and slow["path"] == "generic"
@@ -92,7 +92,7 @@ def test_tiled_diagnostics_round_out_once(pkg, dev, case):
     _, args, cs = _call(pkg, dev, case)
     outs = []
     for general in (False, True):
-        plan = pkg.SrwPlan(*args, chunk_size=cs, diag=True)
+        plan = pkg.SrwPlan(*args, chunk_size=cs, diag=True, tiled=True)
         if general:
             plan._desc.flags |= pkg._capi.SRW_FLAG_NO_FAST
         plan.launch()
