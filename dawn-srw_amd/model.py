@@ -302,12 +302,12 @@ class DawnModel:
         """The layers of a decode step in one library call
         (``srw_dawn_decode_step``), from the embedded rows x [B, D] to the
         final LayerNorm's; None where the call does not apply: more rows than
-        one batch of decode-sized calls, widths the kernels do not take, or
+        one batch of decode-sized calls, no layers, widths the kernels do not take, or
         caches and parameters that are not contiguous float32 on the device."""
         cfg, dev = self.cfg, self.device
         B, D = x.shape
         H, dr, L = cfg.n_heads, cfg.d_route, cfg.n_layers
-        if not (1 <= B and 2 * B <= 128 and D in (128, 384) and D == 64 * H and dr % 16 == 0 and cache_len >= 0):
+        if not (1 <= B and 1 <= L and 2 * B <= 128 and D in (128, 384) and D == 64 * H and dr % 16 == 0 and cache_len >= 0):
             return None
         rt, pool = self.p["router"], self.p["neuron_pool"]
         par = {"proj_attn_w": (rt["proj_attn"]["kernel"], (D, 3 * dr)), "proj_attn_b": (rt["proj_attn"]["bias"], (3 * dr,)),

@@ -96,3 +96,17 @@ def test_general_step_keeps_other_caches(model, dev):
     b = m.decode_step(ids, cK.clone(), cV.clone(), 20)
     assert rel_fro(a[0].cpu(), b[0].cpu()) <= 2e-2
     assert a[1] is strided and rel_fro(strided[..., 20, :].cpu(), b[1][..., 20, :].cpu()) <= 2e-2
+
+
+def test_step_of_a_model_without_layers(pkg, dev):
+    """No layers: the head alone, as the general step computes it."""
+    cfg = pkg.DawnConfig(vocab_size=300, d_model=128, n_layers=0, n_heads=2, max_seq_len=30, d_route=64,
+                         n_qk=300, n_v=500, n_know=1000, max_chunk_size=600)
+    m = pkg.DawnModel(pkg.init_params(cfg, seed=7), cfg, dev)
+    ids, cK, cV = _state(cfg, dev, 3, 4, 8)
+    print("[gpu] decode step, no layers", flush=True)
+    logits, _, _, n = m.decode_step(ids, cK, cV, 4)
+    emb = m.p["token_emb"]["embedding"]
+    x = emb[ids] + m.p["pos_emb"]["embedding"][4]
+    want = torch.nn.functional.layer_norm(x, (128,), m.p["norm"]["scale"], m.p["norm"]["bias"], eps=1e-6) @ emb.T
+    assert n == 5 and torch.equal(logits, want)
