@@ -488,15 +488,23 @@ srw_status_t srw_dawn_decode_step(const srw_dawn_step_t* s, void* stream) {
     if (!wide(s->tensors[i].x) || !wide(s->tensors[i].h) || !s->tensors[i].tau_offset || !wide(s->outs[i].out))
       return SRW_EINVAL;
   }
-  // the SRW calls inside must pass before anything is launched
+  // the SRW calls inside must pass before anything is launched: their own
+  // checks, each on the workspace that it will get
+  for (int32_t i = 0; i < 3; ++i) {
+    // the router's products and the normalised rows are written at once
+    if (s->tensors[i].h == s->tensors[i].x) return SRW_EINVAL;
+    srw::LaunchArgs a;
+    int which = -1;
+    const srw_status_t st = prepare_forward(&s->descs[i], &s->tensors[i], &s->outs[i], i < 2 ? s->ws_qkv : s->ws_know,
+                                            i < 2 ? s->ws_qkv_bytes : s->ws_know_bytes, stream, &a, &which);
+    if (st != SRW_OK) return st;
+  }
   size_t need = 0;
-  srw_status_t st = srw_workspace_size_batch(2, s->descs, &need);
+  const srw_status_t st = srw_workspace_size_batch(2, s->descs, &need);
   if (st != SRW_OK) return st;
   if (need > 0 && (!s->ws_qkv || s->ws_qkv_bytes < need)) return SRW_EWORKSPACE;
-  if ((st = srw_workspace_size_for(&s->descs[2], &s->tensors[2], &need)) != SRW_OK) return st;
-  if (need > 0 && (!s->ws_know || s->ws_know_bytes < need)) return SRW_EWORKSPACE;
   (void)hipGetLastError();
-  return srw::dawn_decode_step(*s, static_cast<hipStream_t>(stream)) == hipSuccess ? SRW_OK : SRW_EHIP;
+  return srw::dawn_decode_step(*s, static_cast<hipStream_t>(stream));
 }
 
 srw_status_t srw_cast_bf16(int32_t n, const float* const* src, void* const* dst, const int64_t* count,

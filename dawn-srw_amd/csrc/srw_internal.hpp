@@ -155,7 +155,7 @@ hipError_t cast_bf16(int n, const float* const* src, uint16_t* const* dst, const
 
 // srw_dawn_decode_step (srw_model.hip), arguments checked.
 bool dawn_step_supports(const srw_dawn_step_t& s);
-hipError_t dawn_decode_step(const srw_dawn_step_t& s, hipStream_t st);
+srw_status_t dawn_decode_step(const srw_dawn_step_t& s, hipStream_t st);
 
 // Tiled-GEMM kernels for wide layers (bf16), see srw_tiled.hip: P = gated
 // product materialised in HBM; d_model and d_route multiples of 64.

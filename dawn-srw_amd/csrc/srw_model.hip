@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kAtThreads) void decode_attn_kernel(AttnParams p) {
 }
 
 template <int NI>
-hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_t st) {
+srw_status_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_t st) {
   const int64_t B = s.B, D = s.d_model, dr = s.d_route;
   auto bf = [](const void* q) { return static_cast<uint16_t*>(const_cast<void*>(q)); };
   auto fl = [](const float* q) { return const_cast<float*>(q); };
@@ -314,7 +314,7 @@ hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_
   const unsigned rt = static_cast<unsigned>((B + 15) / 16);
   float *cur = s.x, *alt = s.x_alt;
   const auto* know_out = static_cast<const uint16_t*>(s.outs[2].out);
-  hipError_t e;
+  srw_status_t e;
   for (int i = 0; i < s.n_layers; ++i) {
     const srw_dawn_layer_t& ly = s.layers[i];
     DenseParams a{};
@@ -346,11 +346,11 @@ hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_
     a.T = B;
     hipLaunchKernelGGL((rows_dense_kernel<NI, true>), dim3(static_cast<unsigned>(a.cols / 16 + 1), rt), dim3(256), 0,
                        st, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (hipGetLastError() != hipSuccess) return SRW_EHIP;
     const bool cached = i > 0;
     for (int k = 0; k < 3; ++k)
       if (cached || (k < 2 ? s.qkv_cached : s.know_cached)) descs[k].flags |= SRW_FLAG_POOL_CACHED;
-    if (srw_forward_batch(2, descs, s.tensors, s.outs, s.ws_qkv, s.ws_qkv_bytes, st) != SRW_OK) return hipErrorUnknown;
+    if ((e = srw_forward_batch(2, descs, s.tensors, s.outs, s.ws_qkv, s.ws_qkv_bytes, st)) != SRW_OK) return e;
     if (s.path_qkv) *s.path_qkv = srw_last_path();
     AttnParams t{};
     t.qk = static_cast<const uint16_t*>(s.outs[0].out);
@@ -365,7 +365,7 @@ hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_
     t.pos = s.pos;
     hipLaunchKernelGGL(decode_attn_kernel, dim3(static_cast<unsigned>(s.n_heads), static_cast<unsigned>(B)),
                        dim3(kAtThreads), 0, st, t);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (hipGetLastError() != hipSuccess) return SRW_EHIP;
     DenseParams o{};
     o.x = s.attn;
     o.w = ly.expand_o;
@@ -373,7 +373,7 @@ hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_
     o.res = cur;
     o.T = B;
     hipLaunchKernelGGL((rows_dense_kernel<NI, false>), dim3(static_cast<unsigned>(D / 16), rt), dim3(256), 0, st, o);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (hipGetLastError() != hipSuccess) return SRW_EHIP;
     DenseParams k{};
     k.x = cur;
     k.ln_scale = ly.norm2_scale;
@@ -392,12 +392,12 @@ hipError_t step(const srw_dawn_step_t& s, const srw_desc_t* descs_in, hipStream_
     k.T = B;
     hipLaunchKernelGGL((rows_dense_kernel<NI, true>), dim3(static_cast<unsigned>(k.cols / 16 + 1), rt), dim3(256), 0,
                        st, k);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (srw_forward(&descs[2], &tk, &s.outs[2], s.ws_know, s.ws_know_bytes, st) != SRW_OK) return hipErrorUnknown;
+    if (hipGetLastError() != hipSuccess) return SRW_EHIP;
+    if ((e = srw_forward(&descs[2], &tk, &s.outs[2], s.ws_know, s.ws_know_bytes, st)) != SRW_OK) return e;
   }
   hipLaunchKernelGGL(final_norm_kernel<NI>, dim3(static_cast<unsigned>((B + 3) / 4)), dim3(256), 0, st, cur, know_out,
                      s.know_scale, s.norm_scale, s.norm_bias, s.normed, B);
-  return hipGetLastError();
+  return hipGetLastError() == hipSuccess ? SRW_OK : SRW_EHIP;
 }
 
 }  // namespace
@@ -407,7 +407,7 @@ bool dawn_step_supports(const srw_dawn_step_t& s) {
          s.d_route % 16 == 0 && s.d_route > 0 && s.B > 0 && s.B <= 65535;
 }
 
-hipError_t dawn_decode_step(const srw_dawn_step_t& s, hipStream_t st) {
+srw_status_t dawn_decode_step(const srw_dawn_step_t& s, hipStream_t st) {
   return s.d_model == 384 ? step<6>(s, s.descs, st) : step<2>(s, s.descs, st);
 }
 

@@ -419,7 +419,9 @@ typedef struct srw_dawn_step {
   const char** path_qkv;        /* host: srw_last_path() after the QK and V calls; or NULL */
 } srw_dawn_step_t;
 /* d_model 128 or 384, heads of 64, d_route a multiple of 16; else
- * SRW_EUNSUPPORTED with nothing launched. */
+ * SRW_EUNSUPPORTED.  The three SRW calls' own checks come first: a call that
+ * srw_forward refuses, or one with h == x (both are written here), returns its
+ * status with nothing launched. */
 srw_status_t srw_dawn_decode_step(const srw_dawn_step_t* step, void* stream);
 
 /* dst[i][k] = bf16(src[i][k]) for k < count[i], i < n: the casts of a fused

@@ -261,6 +261,48 @@ def test_small_pools_keep_their_diagnostics_kernels(C, rows, D, dr, first):
             assert C.workspace_size_for(d, tens) > 0
 
 
+def _decode_step(C, D=128, dr=128, B=4):
+    """A whole srw_dawn_step_t over addresses that nothing reads, and what
+    keeps its host arrays alive."""
+    p = 1 << 20
+    descs = (C.SrwDesc * 3)(*(_desc(C, T=B, d_model=D, d_route=dr, n_routes=r, n_units=n, chunk_size=0,
+                                    stats_mode=C.SRW_STATS_CENTERED) for r, n in ((2, 300), (1, 500), (1, 1000))))
+    tens = (C.SrwTensors * 3)(*(C.SrwTensors(p, 2 * p, p, p, p, p) for _ in range(3)))
+    outs = (C.SrwOutputs * 3)(*(C.SrwOutputs(out=p) for _ in range(3)))
+    layers = (C.SrwDawnLayer * 1)(C.SrwDawnLayer(p, p, p, p, p))
+    s = C.SrwDawnStep(B=B, d_model=D, d_route=dr, max_seq=8, pos=2, n_layers=1, n_heads=D // 64, layers=layers,
+                      descs=descs, tensors=tens, outs=outs, ws_qkv=p, ws_qkv_bytes=1 << 30, ws_know=p,
+                      ws_know_bytes=1 << 30)
+    for name, kind in C.SrwDawnStep._fields_:
+        if kind is ctypes.c_void_p and not getattr(s, name):
+            setattr(s, name, p)
+    return s, descs, tens, outs
+
+
+def test_decode_step_checks_its_calls_before_any_launch(C):
+    """srw_dawn_decode_step: what one of its SRW calls would refuse is refused
+    with that call's status before the first launch, and so is h == x, whose
+    buffer two kernels' results would share."""
+    run = C.load_library().srw_dawn_decode_step
+    for i in range(3):
+        for field in ("emb", "read", "write"):
+            s, _, tens, _ = _decode_step(C)
+            setattr(tens[i], field, None)
+            assert run(ctypes.byref(s), None) == C.SRW_EINVAL, (i, field)
+        s, _, tens, _ = _decode_step(C)
+        tens[i].h = tens[i].x
+        assert run(ctypes.byref(s), None) == C.SRW_EINVAL, i
+        s, descs, _, _ = _decode_step(C)
+        descs[i].stats_mode, descs[i].flags = C.SRW_STATS_GRAM, C.SRW_FLAG_NO_FAST
+        assert run(ctypes.byref(s), None) == C.SRW_EUNSUPPORTED, i
+    for field in ("ws_qkv_bytes", "ws_know_bytes"):
+        s, *_ = _decode_step(C)
+        setattr(s, field, 256)
+        assert run(ctypes.byref(s), None) == C.SRW_EWORKSPACE, field
+    s, *_ = _decode_step(C, D=192, dr=64)
+    assert run(ctypes.byref(s), None) == C.SRW_EUNSUPPORTED
+
+
 def test_status_strings(C):
     lib = C.load_library()
     for s in range(6):
