@@ -49,9 +49,11 @@ def _both(m, monkeypatch, ids, cK, cV, n):
     return a, b
 
 
-# one row, ragged row tiles, the largest batch; no cached position, one group's
-# first, one round of groups and its neighbours, more than one chunk, the last
-@pytest.mark.parametrize("B,n", [(1, 0), (3, 1), (17, 31), (16, 32), (33, 33), (64, 257), (5, 299)])
+# one row, ragged row tiles, the largest batch of one launch per stage and
+# larger ones; no cached position, one group's first, one round of groups and
+# its neighbours, more than one chunk, the last
+@pytest.mark.parametrize("B,n", [(1, 0), (3, 1), (17, 31), (16, 32), (33, 33), (64, 257), (5, 299), (65, 40),
+                                 (96, 12), (200, 33)])
 def test_native_step_matches_general(model, dev, monkeypatch, B, n):
     cfg, m = model
     print(f"[gpu] native decode step D{cfg.d_model} B{B} len{n}", flush=True)
