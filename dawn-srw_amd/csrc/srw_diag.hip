@@ -272,8 +272,8 @@ __global__ __launch_bounds__(256) void diag_rows_units_kernel(DsumParams p) {
       const bool dead = p.ud[n * SRW_UDIAG_COUNT + SRW_UDIAG_GATE_MAX] < p.dead_threshold;
       v[DS_PN] += pn;
       v[DS_PN2] += static_cast<double>(pn) * pn;
-      // relu(-pn) * dead; a NaN mean stays one, also times 0 (v41:548-552)
-      v[DS_PEN] += pn != pn ? pn : (dead && pn < 0.f ? -pn : 0.f);
+      // relu(-pn) * dead, a product: a NaN or -inf mean gives NaN also times 0 (v41:548-552)
+      v[DS_PEN] += (pn != pn ? pn : (pn < 0.f ? -pn : 0.f)) * (dead ? 1.f : 0.f);
       v[DS_DEAD] += dead ? 1.0 : 0.0;
     }
   }

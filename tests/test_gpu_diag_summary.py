@@ -79,6 +79,34 @@ def test_summary_keeps_nan(pkg, dev):
     assert not torch.isnan(got[13])
 
 
+@pytest.mark.parametrize("gate,R", [("v41", 1), ("v41", 2), ("gelu_v401", 2)])
+def test_summary_of_infinities(pkg, dev, gate, R):
+    """An infinity or NaN in any column comes out where the torch form gives
+    one (relu(inf) times a dead unit's 0 among them), and nowhere else."""
+    from dawn_srw_amd import srw
+    B, S, N = 1, 70, 60
+    print(f"[gpu] diag summary infinities {gate} R{R}", flush=True)
+    v401 = gate != "v41"
+    for v in (float("inf"), float("-inf"), float("nan")):
+        for name, at in ([("token_diag", (33, 0, k)) for k in range(14)] + [("gate_sum", (33, 0))]
+                         + [("unit_diag", (u, k)) for u in (7, 8) for k in (0, 1)]):
+            plan = _plan(pkg, dev, B, S, N, R, gate)
+            g = torch.Generator(device=dev).manual_seed(5)
+            plan.token_diag.uniform_(0.5, 2.0, generator=g)
+            plan.gate_sum.uniform_(0.5, 5.0, generator=g)
+            plan.n_active.random_(1, N + 1, generator=g)
+            plan.unit_diag.normal_(generator=g)
+            plan.unit_diag[7, 1], plan.unit_diag[8, 1] = 0.0, 1.0  # a dead unit and one that is not
+            getattr(plan, name)[at] = v
+            res = plan.results()
+            want = srw._diag_tuple_v401(res, N, B, S, R) if v401 else srw._diag_tuple(res, N, B, S, R, 0.01)
+            got = srw._fused_diag(plan, N, B, S, R, 0.0 if v401 else 0.01, v401)
+            for i, (a, b) in enumerate(zip(got, want)):
+                assert torch.equal(torch.isnan(a), torch.isnan(b)), (v, name, at, i, a.flatten()[:1], b.flatten()[:1])
+                inf = torch.isinf(b)
+                assert torch.equal(torch.isinf(a), inf) and torch.equal(a[inf], b[inf]), (v, name, at, i)
+
+
 def test_cast_bf16_bit_equal(pkg, dev):
     from dawn_srw_amd import layer
     g = torch.Generator(device=dev).manual_seed(3)
