@@ -1183,9 +1183,8 @@ __device__ __attribute__((always_inline)) inline void write_body(const TWritePar
   else
     store(std::false_type{});
 }
-template <int NBF, bool MAYROUND = false>
 __global__ __launch_bounds__(kGThreads) void tiled_write_kernel(TWriteParams p) {
-  write_body<NBF, MAYROUND>(p, blockIdx.x);
+  write_body<4, false>(p, blockIdx.x);
 }
 // Several independent products in one launch (the backward's five gradient
 // contractions): group i owns workgroups [start[i], start[i + 1]), each
@@ -1360,8 +1359,9 @@ hipError_t set_lds(const void* fn, int bytes = kGemmLds) {
 }  // namespace
 
 // The operand loaders keep each lane's byte offset within a 256-row tile in
-// 32 bits: 256 rows of ld bf16 elements must stay below 4 GiB (ld = N or T
-// padded to 64 for the stored [., N64] / [., T64] arrays).
+// 32 bits: 256 rows of ld bf16 elements must stay below 4 GiB (ld = N padded
+// to 64 for the stored [., N64] arrays).  The backward refuses more rows than
+// that too, 8.4 M of them: a limit of the call, no kernel's.
 static bool tile_offsets_fit(int64_t ld) { return 256 * ((ld + kNAlign - 1) / kNAlign * kNAlign) * 2 < (int64_t(1) << 32); }
 
 // Diagnostics come from the stored scores before the gate kernel writes P
@@ -1495,7 +1495,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   for (const void* fn : {reinterpret_cast<const void*>(tiled_stats_kernel),
                          reinterpret_cast<const void*>(tiled_gate_kernel<false>),
                          reinterpret_cast<const void*>(tiled_gate_kernel<true>),
-                         reinterpret_cast<const void*>(tiled_write_kernel<4>)})
+                         reinterpret_cast<const void*>(tiled_write_kernel)})
     if ((e = set_lds(fn)) != hipSuccess) return e;
 
   if (!(d.flags & SRW_FLAG_POOL_CACHED) && !tiled_sparse(d)) {  // (the sparse path gathers W's rows)
@@ -1592,7 +1592,7 @@ hipError_t tiled_forward(const LaunchArgs& a) {
   wp.RT = g.RT;
   wp.DT = g.DT;
   const unsigned grid_w = static_cast<unsigned>(8 * g.DT * ((static_cast<int64_t>(g.RT) * g.S + 7) / 8));
-  hipLaunchKernelGGL(tiled_write_kernel<4>, dim3(grid_w), dim3(kGThreads), kGemmLds, a.stream, wp);
+  hipLaunchKernelGGL(tiled_write_kernel, dim3(grid_w), dim3(kGThreads), kGemmLds, a.stream, wp);
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
   hipLaunchKernelGGL(tiled_tok_sum_kernel, dim3(static_cast<unsigned>((g.Tv + 63) / 64)), dim3(256), 0, a.stream,
@@ -2203,6 +2203,11 @@ __global__ __launch_bounds__(TH, TH == 256 ? 4 : TH / 128) void bwd_row_kernel(R
 
 // Units up to which a row fits the registers of 512 threads (twelve a chunk and
 // route, 128 a thread without spilling, two workgroups a CU); longer rows: two passes.
+// No line in the tokens: with one workgroup a token a short call leaves CUs idle, but
+// the passes' launches cost as much.  srw_backward, rows kernel / two passes in us:
+// N = 25 200 at 1, 64, 256, 512 tokens 140 / 136, 145 / 146, 169 / 183, 221 / 245;
+// N = 3 000 71 / 79, 80 / 87, 85 / 92, 108 / 117; paired, N = 12 000 101 / 101,
+// 115 / 117, 125 / 137, 152 / 173 (v4.0.1 alike).
 constexpr int64_t row_max_units(int routes) { return 8 * 512 * (routes == 2 ? 3 : 7); }
 template <int RT, bool GL>
 void launch_rows(const RowParams& q, hipStream_t st) {
@@ -2457,7 +2462,7 @@ __global__ __launch_bounds__(256) void bwd_pad_kernel(PadParams p) {
 struct BGemm {
   int64_t M, Nc, K;  // out [M, Nc] = A [M, K] . B [Nc, K]^T
   int RT, DT, spc;
-  int nbf;           // tile width 64 nbf (tiled_write_kernel<nbf>)
+  int nbf;           // tile width 64 nbf (tiled_write_batch_kernel<nbf>, tiled_grad_kernel<nbf>)
 };
 
 BGemm bgemm(int64_t M, int64_t Nc, int64_t K) {
