@@ -373,8 +373,9 @@ struct NoHook {
 // a row, the 16-byte piece q of row r in slot q ^ (r & 15).  An accumulator
 // holds four consecutive units per lane, 8 bytes in each of 32 rows: straight
 // to memory, every access touches 32 lines and every line is touched eight
-// times; through here each access is four rows' whole lines, streamed past L2
-// (the array is larger than it).  T = 16 384, N = 100 000, D = dr = 1 024:
+// times; through here each access is four rows' whole lines (stored
+// non-temporally; plain stores measure the same, within 0.5%, for arrays of 0.1 MB
+// to 1 GB).  T = 16 384, N = 100 000, D = dr = 1 024:
 // score kernel 4 002 -> 3 477 us (2 720 without an epilogue), gate kernel,
 // whose scores arrive under the last blocks' products, 5 432 -> 4 787.
 struct RowPatch {
